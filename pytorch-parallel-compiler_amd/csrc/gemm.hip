@@ -4,14 +4,17 @@
 // A and W are K-contiguous ("NT"), which is exactly the operand layout MFMA
 // wants: every lane feeds 8 consecutive k values of one row.
 //
-// Tiling: a workgroup of WM x WN waves computes a (WM*TM) x (WN*TN) tile of C;
-// each wave owns a TM x TN sub-tile made of 16x16 MFMA tiles accumulated in
-// fp32.  K advances in steps of 32.  A and W tiles are staged in LDS (double
+// Three kernels share a problem's sizes between them (launch_gemm_t): gemm_kernel here for small
+// problems, the 128 x 128 / 64 x 64 tile kernel of gemm_tile.hip, and the persistent XL kernels
+// here for large 16-bit ones.
+//
+// gemm_kernel: a workgroup of 2 x 2 waves computes a 32 x 32 tile of C, each wave one 16x16 MFMA
+// tile accumulated in fp32.  K advances in steps of 32.  A and W tiles are staged in LDS (double
 // buffered: the next K-step is fetched into registers while the current one
 // feeds the MFMAs); rows are padded by 16 bytes so the 16-byte fragment reads
 // of a quarter-wave hit 64 distinct banks.
 //
-// bf16 uses v_mfma_f32_16x16x32_bf16 (one instruction per K-step of 32);
+// There bf16 uses v_mfma_f32_16x16x32_bf16 (one instruction per K-step of 32);
 // fp32 uses v_mfma_f32_16x16x4_f32 with the K-step permuted so that lane
 // group g (lanes 16g..16g+15) contributes k = 8g .. 8g+7 over eight
 // instructions -- a reordering of the k summation only.
@@ -29,17 +32,13 @@ namespace wc {
 namespace {
 
 constexpr int kBK = 32;
-
-template <typename TA> struct Frag;
-template <> struct Frag<bf16> { typedef bf16x8 type; };
-template <> struct Frag<float> { typedef f32x4 type; };  // two per K-step
-template <> struct Frag<f16> { typedef bf16x8 type; };    // raw 16-bit lanes, as bf16
-
+constexpr int kSmallTile = 32;              // rows and columns of a small-tile workgroup
 
 __device__ __forceinline__ float relu_f(float v) { return v > 0.f ? v : 0.f; }
 
-template <typename TA, typename TC, typename TB, int TM, int TN, int WM, int WN, bool VEC>
-__global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(GemmParams p) {
+template <typename TA, typename TC, typename TB, bool VEC>
+__global__ __launch_bounds__(256) void gemm_kernel(GemmParams p) {
+  constexpr int TM = 16, TN = 16, WM = 2, WN = 2;
   constexpr int NT = WM * WN * 64;
   constexpr int BM = WM * TM, BN = WN * TN;
   constexpr int ES = sizeof(TA);
@@ -227,187 +226,6 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(GemmParams p) {
         cbase[off] = from_f32<TC>(v);
       }
     }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Large-tile bf16 kernel.  A workgroup of WM x WN waves computes a
-// (WM*FM*16) x (WN*FN*16) tile; K advances in tiles of 64 staged through a
-// double-buffered LDS ring (each thread moves 16-byte chunks global ->
-// registers -> LDS; the next tile's loads are in flight during the current
-// tile's 2 x FM x FN MFMAs).  The epilogue goes through LDS as well: each wave
-// parks a 16-row strip of its fp32 accumulators, reads it back row-major and
-// applies bias / residual / ReLU with 8- or 16-byte stores along rows.
-// ---------------------------------------------------------------------------
-constexpr int kBigBK = 64;
-constexpr int kBigPitch = kBigBK + 8;          // bf16 elements per LDS row (144 bytes)
-
-template <int WM, int WN, int FM, int FN>
-struct BigCfg {
-  static constexpr int NT = WM * WN * 64;
-  static constexpr int BM = WM * FM * 16, BN = WN * FN * 16;
-  static constexpr int CH = (BM + BN) * (kBigBK / 8);        // 16-byte chunks per stage
-  static constexpr int CPT = CH / NT;                       // chunks per thread
-  static constexpr int STAGE = (BM + BN) * kBigPitch;       // bf16 elements per stage
-  static constexpr int EPI_PITCH = FN * 16 + 4;             // floats per epilogue row
-  static constexpr size_t LDS_MAIN = 2 * STAGE * sizeof(bf16);
-  static constexpr size_t LDS_EPI = static_cast<size_t>(WM * WN) * 16 * EPI_PITCH * sizeof(float);
-  static constexpr size_t LDS = LDS_MAIN > LDS_EPI ? LDS_MAIN : LDS_EPI;
-  static_assert(CH % NT == 0, "chunks must divide evenly");
-};
-
-template <typename TA, typename TC, typename TB, int WM, int WN, int FM, int FN>
-__global__ __launch_bounds__(WM* WN * 64) void gemm_big_kernel(GemmParams p) {
-  using C = BigCfg<WM, WN, FM, FN>;
-  constexpr int NT = C::NT, BM = C::BM, BN = C::BN, CPT = C::CPT;
-  extern __shared__ __attribute__((aligned(16))) bf16 big_smem[];
-
-  const int tiles_per_model = p.tiles_m * p.tiles_o;
-  const int nblk = p.n * tiles_per_model;
-  int bid = blockIdx.x;
-  if (p.remap) bid = (blockIdx.x & 7) * (nblk >> 3) + (blockIdx.x >> 3);
-  const int mdl = bid / tiles_per_model;
-  const int rem = bid - mdl * tiles_per_model;
-  const int to = rem / p.tiles_m;
-  const int tm = rem - to * p.tiles_m;
-  const int m0 = tm * BM, o0 = to * BN;
-
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  const int wm = wave / WN, wn = wave - (wave / WN) * WN;
-
-  const bf16* abase = static_cast<const bf16*>(p.a) + static_cast<int64_t>(mdl) * p.a_sn;
-  const bf16* wbase = static_cast<const bf16*>(p.w) + static_cast<int64_t>(mdl) * p.w_sn;
-
-  // staging: chunk c = tid + q*NT; rows [0, BM) are A, [BM, BM+BN) are W
-  const bf16* src[CPT];
-  int dst[CPT];
-#pragma unroll
-  for (int q = 0; q < CPT; ++q) {
-    const int c = tid + q * NT;
-    const int r = c >> 3, kc = (c & 7) * 8;
-    dst[q] = r * kBigPitch + kc;
-    src[q] = nullptr;
-    if (r < BM) {
-      const int gm = m0 + r;
-      if (gm < p.m) {
-        const uint32_t outer = fdiv(static_cast<uint32_t>(gm), p.a_ri);
-        const uint32_t inner = gm - outer * p.a_ri.d;
-        src[q] = abase + static_cast<int64_t>(outer) * p.a_so + static_cast<int64_t>(inner) * p.a_si + kc;
-      }
-    } else {
-      const int go = o0 + (r - BM);
-      if (go < p.o) src[q] = wbase + static_cast<int64_t>(go) * p.k + kc;
-    }
-  }
-  uint4 stg[CPT];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int q = 0; q < CPT; ++q) {
-      const int kk = k0 + (dst[q] % kBigPitch);
-      stg[q] = (src[q] && kk < p.k) ? *reinterpret_cast<const uint4*>(src[q] + k0) : make_uint4(0, 0, 0, 0);
-    }
-  };
-  auto stash = [&](int stage) {
-    bf16* base = big_smem + stage * C::STAGE;
-#pragma unroll
-    for (int q = 0; q < CPT; ++q) *reinterpret_cast<uint4*>(base + dst[q]) = stg[q];
-  };
-
-  f32x4 acc[FM][FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int ktiles = (p.k + kBigBK - 1) / kBigBK;
-  fetch(0);
-  stash(0);
-  __syncthreads();
-  const int fr = lane & 15, fk = (lane >> 4) * 8;
-  for (int kt = 0; kt < ktiles; ++kt) {
-    const int stage = kt & 1;
-    if (kt + 1 < ktiles) fetch((kt + 1) * kBigBK);
-    const bf16* as = big_smem + stage * C::STAGE + (wm * FM * 16 + fr) * kBigPitch + fk;
-    const bf16* bs = big_smem + stage * C::STAGE + (BM + wn * FN * 16 + fr) * kBigPitch + fk;
-#pragma unroll
-    for (int kk = 0; kk < kBigBK; kk += 32) {
-      bf16x8 af[FM], bfr[FN];
-#pragma unroll
-      for (int i = 0; i < FM; ++i) af[i] = *reinterpret_cast<const bf16x8*>(as + i * 16 * kBigPitch + kk);
-#pragma unroll
-      for (int j = 0; j < FN; ++j) bfr[j] = *reinterpret_cast<const bf16x8*>(bs + j * 16 * kBigPitch + kk);
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-          acc[i][j] = mma16<TA>(af[i], bfr[j], acc[i][j]);
-    }
-    if (kt + 1 < ktiles) stash(stage ^ 1);
-    __syncthreads();
-  }
-
-  // ---- epilogue through LDS: one 16-row strip of the wave's tile at a time ----
-  constexpr int EP = C::EPI_PITCH;
-  constexpr int COLS = FN * 16;
-  constexpr int LPR = COLS / 4;                  // lanes per row (4 columns each)
-  constexpr int RPI = 64 / LPR;                  // rows per read instruction
-  float* ep = reinterpret_cast<float*>(big_smem) + wave * 16 * EP;
-  const TB* bias = p.bias ? static_cast<const TB*>(p.bias) + static_cast<int64_t>(mdl) * p.b_sn : nullptr;
-  TC* cbase = static_cast<TC*>(p.c) + static_cast<int64_t>(mdl) * p.c_sn;
-  const TC* rbase = p.r ? static_cast<const TC*>(p.r) + static_cast<int64_t>(mdl) * p.r_sn : nullptr;
-  const int lc = (lane % LPR) * 4;               // this lane's 4 columns within the strip
-  const int col0 = o0 + wn * COLS + lc;
-  const bool vec4 = (p.o & 3) == 0;
-  float bv[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) bv[e] = (bias && col0 + e < p.o) ? to_f32(bias[col0 + e]) : 0.f;
-#pragma unroll
-  for (int i = 0; i < FM; ++i) {
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) ep[((lane >> 4) * 4 + e) * EP + j * 16 + fr] = acc[i][j][e];
-    __builtin_amdgcn_s_waitcnt(0xc07f);          // lgkmcnt(0): this wave's strip is in LDS
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int rr = 0; rr < 16; rr += RPI) {
-      const int lr = rr + lane / LPR;
-      const int row = m0 + wm * FM * 16 + i * 16 + lr;
-      const f32x4 v4 = *reinterpret_cast<const f32x4*>(ep + lr * EP + lc);
-      if (row < p.m && col0 < p.o) {
-        const uint32_t outer = fdiv(static_cast<uint32_t>(row), p.c_ri);
-        const uint32_t inner = row - outer * p.c_ri.d;
-        const int64_t off = static_cast<int64_t>(outer) * p.c_so + static_cast<int64_t>(inner) * p.c_si + col0;
-        float v[4] = {v4[0] + bv[0], v4[1] + bv[1], v4[2] + bv[2], v4[3] + bv[3]};
-        if (rbase) {
-          const int64_t roff = static_cast<int64_t>(outer) * p.r_so + static_cast<int64_t>(inner) * p.r_si + col0;
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (col0 + e < p.o) v[e] += to_f32(rbase[roff + e]);
-        }
-        if (p.act == WC_ACT_RELU)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = relu_f(v[e]);
-        if (vec4 && col0 + 3 < p.o) {
-          if constexpr (sizeof(TC) == 4) {
-            *reinterpret_cast<f32x4*>(cbase + off) = f32x4{v[0], v[1], v[2], v[3]};
-          } else {
-            typedef TC tc4 __attribute__((ext_vector_type(4)));
-            tc4 o4;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o4[e] = from_f32<TC>(v[e]);
-            *reinterpret_cast<tc4*>(cbase + off) = o4;
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (col0 + e < p.o) cbase[off + e] = from_f32<TC>(v[e]);
-        }
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(0xc07f);
-    __builtin_amdgcn_wave_barrier();
   }
 }
 
@@ -1135,39 +953,18 @@ int32_t launch_xl(GemmParams p, hipStream_t st) {
   return check_launch("wc_grouped_gemm");
 }
 
-template <typename TA, typename TC, typename TB, int WM, int WN, int FM, int FN>
-int32_t launch_big(GemmParams p, hipStream_t st) {
-  using C = BigCfg<WM, WN, FM, FN>;
-  p.tiles_m = static_cast<int>(cdiv(p.m, C::BM));
-  p.tiles_o = static_cast<int>(cdiv(p.o, C::BN));
+template <typename TA, typename TC, typename TB>
+int32_t launch_small(GemmParams p, bool vec, hipStream_t st) {
+  p.tiles_m = static_cast<int>(cdiv(p.m, kSmallTile));
+  p.tiles_o = static_cast<int>(cdiv(p.o, kSmallTile));
   const int64_t nblk = static_cast<int64_t>(p.n) * p.tiles_m * p.tiles_o;
   if (nblk >= 0x7fffffffll) return set_error(WC_ERR_LIMIT, "wc_grouped_gemm: too many tiles");
   p.remap = (nblk % 8 == 0) ? 1 : 0;
-  auto kern = gemm_big_kernel<TA, TC, TB, WM, WN, FM, FN>;
-  if (C::LDS > 64 * 1024) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(C::LDS));
-    if (e != hipSuccess)
-      return set_error(static_cast<int32_t>(e), "wc_grouped_gemm: LDS of %zu bytes refused: %s", C::LDS,
-                       hipGetErrorString(e));
-  }
-  kern<<<dim3(static_cast<uint32_t>(nblk)), dim3(C::NT), C::LDS, st>>>(p);
-  return check_launch("wc_grouped_gemm");
-}
-
-template <typename TA, typename TC, typename TB, int TM, int TN, int WM, int WN>
-int32_t launch_cfg(GemmParams p, bool vec, hipStream_t st) {
-  constexpr int BM = WM * TM, BN = WN * TN;
-  p.tiles_m = static_cast<int>(cdiv(p.m, BM));
-  p.tiles_o = static_cast<int>(cdiv(p.o, BN));
-  const int64_t nblk = static_cast<int64_t>(p.n) * p.tiles_m * p.tiles_o;
-  if (nblk >= 0x7fffffffll) return set_error(WC_ERR_LIMIT, "wc_grouped_gemm: too many tiles");
-  p.remap = (nblk % 8 == 0) ? 1 : 0;
-  const dim3 grid(static_cast<uint32_t>(nblk)), block(WM * WN * 64);
+  const dim3 grid(static_cast<uint32_t>(nblk)), block(256);
   if (vec)
-    gemm_kernel<TA, TC, TB, TM, TN, WM, WN, true><<<grid, block, 0, st>>>(p);
+    gemm_kernel<TA, TC, TB, true><<<grid, block, 0, st>>>(p);
   else
-    gemm_kernel<TA, TC, TB, TM, TN, WM, WN, false><<<grid, block, 0, st>>>(p);
+    gemm_kernel<TA, TC, TB, false><<<grid, block, 0, st>>>(p);
   return check_launch("wc_grouped_gemm");
 }
 
@@ -1194,21 +991,31 @@ bool xl_shape_ok(const GemmParams& p) {
   return a_end < lim && w_end < lim && c_end < lim && r_end < lim;
 }
 
+// Which kernel runs a problem, by the tiles it is made of (times in us, one launch in a graph of
+// back-to-back launches, n models of m x k x o):
+//  - the persistent XL kernel when its 256 x 256 tiles cover the CUs and its alignments hold
+//    (bf16 16 x 2048 x 128 x 1024: 19.0 against 29.8 with 128 x 128 tiles);
+//  - 128 x 128 tiles from two rounds of CUs on, unless the padding of short m or o wastes them
+//    (fp32 32 x 1024 x 256 x 256, 512 tiles: 34.4 against 37.7 with 64 x 64; 16 x 512 x 256 x 512,
+//    256 tiles: 22.6 against 21.9);
+//  - 64 x 64 tiles while they cover the CUs (fp32 16 x 256 x 256 x 256, 256 tiles: 10.3 against
+//    11.7 with 32 x 32; 8 x 256 x 512 x 256, 128 tiles: 15.9 against 12.1).  Rows or columns that
+//    fill at most half of a 64-wide tile leave fp32 to the small tiles (64 x 16 x 256 x 1024:
+//    20.4 against 18.3).  16-bit problems cost 32 x 32 tiles a barrier per 32 values of k, so
+//    they take 64 x 64 tiles from the first on (1 x 64 x 2048 x 64: 15.2 against 20.2) unless k
+//    is short (64 x 64 x 64 x 64: 4.4 against 3.8);
+//  - 32 x 32 tiles otherwise: the most workgroups in flight and the fewest dependent MFMAs.
 template <typename TA, typename TC, typename TB>
 int32_t launch_gemm_t(const GemmParams& p, bool vec, hipStream_t st) {
-  if constexpr (sizeof(TA) == 2) {
-    const int64_t tiles256 = static_cast<int64_t>(p.n) * cdiv(p.m, 256) * cdiv(p.o, 256);
-    if constexpr (sizeof(TC) == 2)
-      if (vec && tiles256 >= 256 && xl_shape_ok<TC>(p)) return launch_xl<TA, TB>(p, st);
-    if (vec && tiles256 >= 256) return launch_big<TA, TC, TB, 2, 4, 8, 4>(p, st);
+  auto tiles = [&](int b) { return static_cast<int64_t>(p.n) * cdiv(p.m, b) * cdiv(p.o, b); };
+  if constexpr (sizeof(TA) == 2 && sizeof(TC) == 2) {
+    if (vec && tiles(256) >= 256 && xl_shape_ok<TC>(p)) return launch_xl<TA, TB>(p, st);
   }
-  const int64_t tiles128 = static_cast<int64_t>(p.n) * cdiv(p.m, 128) * cdiv(p.o, 128);
-  if (tiles128 >= 512) return launch_cfg<TA, TC, TB, 64, 64, 2, 2>(p, vec, st);
-  const int64_t tiles64 = static_cast<int64_t>(p.n) * cdiv(p.m, 64) * cdiv(p.o, 64);
-  if (tiles64 >= 1024) return launch_cfg<TA, TC, TB, 32, 32, 2, 2>(p, vec, st);
-  // small problems are latency-bound: 16 x 16 wave tiles give each wave the
-  // fewest dependent MFMAs and the most workgroups in flight
-  return launch_cfg<TA, TC, TB, 16, 16, 2, 2>(p, vec, st);
+  const int64_t t128 = tiles(128), t64 = tiles(64), t32 = tiles(32);
+  if (t128 >= 512 && t128 * 7 <= t64 * 2) return gemm_tile<TA, TC, TB>(p, 128, st);
+  if (sizeof(TA) == 4 ? (t64 >= 192 && t32 * 2 > t64 * 5) : (t64 >= 256 || p.k > 64))
+    return gemm_tile<TA, TC, TB>(p, 64, st);
+  return launch_small<TA, TC, TB>(p, vec, st);
 }
 
 }  // namespace

@@ -30,7 +30,13 @@ struct GemmParams {
   // so a stray offset is dropped by the hardware instead of reaching other memory)
   FastDiv fd_ks, fd_tpm, fd_tm;
   int32_t c_bytes, r_bytes;
+  int vec_c;                   // tile kernel only: C and R rows take 16-byte accesses
 };
+
+// The tile kernel (gemm_tile.hip), with 128 x 128 or 64 x 64 tiles (bm); any sizes, strides and
+// alignments.
+template <typename TA, typename TC, typename TB>
+int32_t gemm_tile(const GemmParams& p, int bm, hipStream_t st);
 
 // dtype: A/W element type; out_dtype: WC_F32 or dtype; bias_dtype: WC_F32 or dtype.
 int32_t grouped_gemm(const GemmParams& p, int32_t dtype, int32_t out_dtype, int32_t bias_dtype,
