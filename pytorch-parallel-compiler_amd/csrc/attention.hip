@@ -5,7 +5,12 @@
 // layout the projection GEMMs produce (head h = columns [h*Dh, (h+1)*Dh)), so no
 // head-major copies are made.
 //
-// Per workgroup: one (model*batch, head) pair and a tile of 128 queries, four
+// Three kernels here, next to the streaming 16-bit one (attention_stream.hip): attn_kernel, the
+// general one (fp32, masks, head dims and rows the others do not take), attn_res_kernel (bf16,
+// head dim 32, K and V resident in LDS) and attn_qkv_kernel (the same with the projections
+// inside).
+//
+// attn_kernel, per workgroup: one (model*batch, head) pair and a tile of 128 queries, four
 // waves of 32 queries each.  For every tile of 64 keys:
 //   S^T = K Q^T          (MFMA; the output layout puts 4 consecutive keys of
 //                         one query in each lane)
@@ -17,32 +22,12 @@
 // K tiles are staged in LDS row-major, V tiles transposed (V^T [Dh][keys]); the
 // next tile is fetched into registers while the current one is processed.
 // Scores are scaled by log2(e)/sqrt(Dh) so the exponentials are v_exp_f32 (2^x).
-#include "wc_common.h"
+#include "wc_attn.h"
 
 #include <type_traits>
 
 namespace wc {
 namespace {
-
-struct AttnParams {
-  int nb, heads, sq, skv, causal, q_tiles;
-  float scale_log2;
-  const void* q;
-  int64_t q_sb, q_ss;
-  const void* k;
-  int64_t k_sb, k_ss;
-  const void* v;
-  int64_t v_sb, v_ss;
-  void* o;
-  int64_t o_sb, o_ss;
-  // additive fp32 mask, element (nb, head, query, key) at nb*m_sb + head*m_sh + query*m_sq + key
-  // (general kernel only; NULL = none)
-  const float* mask;
-  int64_t m_sb, m_sh, m_sq;
-  // head dims other than the kernel's own (attn_kernel with GEN): the true head dim, and the
-  // first head-dim column of the output chunk this launch computes
-  int dh, oc0;
-};
 
 constexpr int kAttnThreads = 256;
 constexpr int kBQ = 128;   // queries per workgroup (32 per wave)
@@ -382,7 +367,7 @@ void attn_kernel(AttnParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Resident-KV kernel (bf16, head dim 32 or 64, K and V of one head fit in LDS).
+// Resident-KV kernel (bf16, head dim 32, full attention, K and V of one head fit in LDS).
 // One workgroup per (model*batch, head, tile of W*64 queries).  K (row-major,
 // rows padded by 16 bytes) and V^T ([dh][key], rows padded by 8 bytes) of every
 // key are staged in LDS once, so the key loop has no barriers.  Each wave owns
@@ -428,9 +413,7 @@ inline size_t res_lds_bytes(int dh, int skvp) {
   return (static_cast<size_t>(skvp) * (dh + 8) + static_cast<size_t>(dh) * (skvp + 4)) * sizeof(bf16);
 }
 
-// The key loop of attn_res_kernel as functions, for attn_qkv_kernel.  attn_res_kernel keeps its
-// own inline copy: its causal variant compiled through these functions takes 136 VGPRs
-// instead of 121, which costs a wave per SIMD.
+// The key loop of attn_res_kernel as functions, with a causal form, for attn_qkv_kernel.
 //
 // One wave's two 32-query blocks in the resident-KV key loop: the Q^T fragments (B operand of
 // S^T = K Q^T, pre-scaled by scale * log2(e)), the row of -base that the extra k-step adds
@@ -571,8 +554,8 @@ __device__ __forceinline__ void res_store_o(const ResRows<NKS, DT>& r, const int
   }
 }
 
-template <int DH, int W, bool CAUSAL>
-__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W == 4 ? 2 : 1))) void attn_res_kernel(AttnParams p, int skvp) {
+template <int DH, int W>
+__global__ __launch_bounds__(W * 64) void attn_res_kernel(AttnParams p, int skvp) {
   constexpr int KP = res_kpitch<DH>();
   constexpr int NKS = DH / 16;                       // 16-dim k-steps of S^T = K Q^T
   constexpr int DT = DH / 32;                        // 32-row tiles of O^T
@@ -626,8 +609,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W == 4 ?
 
   // ---- this wave's queries and their Q^T fragments (B operand of S^T) ----
   // first query rows of the wave's two 32-query blocks: blocks wave and 2W - 1 - wave of
-  // the tile's 2W, so that under a causal mask every wave has the same number of key
-  // blocks to process (a block is skipped for the query block it lies wholly after)
+  // the tile's 2W
   const int qt0 = qt * (W * 64);
   const int qrow[2] = {qt0 + wave * 32, qt0 + (2 * W - 1 - wave) * 32};
   bf16x8 qf[2][NKS];
@@ -669,12 +651,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W == 4 ?
       for (int e = 0; e < 16; ++e) oacc[b][d][e] = 0.f;
   // base[b]: the bf16 value subtracted from this row's exponents (0 until the first block sets it)
   float base[2] = {0.f, 0.f}, lrun[2] = {0.f, 0.f};
-  int nkb = skvp / 32;
-  if (CAUSAL) {
-    const int qmax = qrow[1] + 31;                  // qrow[1] >= qrow[0]
-    const int last = (qmax < p.sq ? qmax : p.sq - 1) / 32 + 1;
-    nkb = last < nkb ? last : nkb;
-  }
+  const int nkb = skvp / 32;
   // one 32-key block: both query blocks' scores first (their MFMA latency hides
   // behind the first block's softmax), then per query block softmax and P V
   auto key_block = [&](int kbk, auto mask_tag, bool first) {
@@ -701,7 +678,6 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W == 4 ?
     f32x16 s[2];
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-      if (CAUSAL && key0 > qrow[b] + 31) continue;
 #pragma unroll
       for (int e = 0; e < 16; ++e) s[b][e] = 0.f;
 #pragma unroll
@@ -710,13 +686,11 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W == 4 ?
     }
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-      if (CAUSAL && key0 > qrow[b] + 31) continue;
       if constexpr (MASK) {
-        const int q = qrow[b] + l32;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int key = key0 + (r >> 2) * 8 + 4 * hf + (r & 3);
-          if (key >= p.skv || (CAUSAL && key > q)) s[b][r] = -INFINITY;
+          if (key >= p.skv) s[b][r] = -INFINITY;
         }
       }
       // tree reductions keep the dependency chains short
@@ -770,20 +744,9 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W == 4 ?
   };
   using masked = std::integral_constant<bool, true>;
   using unmasked = std::integral_constant<bool, false>;
-  if (CAUSAL) {
-    // only the blocks on a query block's diagonal, or past the last key, need the mask
-    for (int kbk = 0; kbk < nkb; ++kbk) {
-      const int key0 = kbk * 32;
-      if ((key0 + 31 > qrow[0] && key0 <= qrow[0] + 31) || key0 + 31 > qrow[1] || key0 + 32 > p.skv)
-        key_block(kbk, masked{}, kbk == 0);
-      else
-        key_block(kbk, unmasked{}, kbk == 0);
-    }
-  } else {
-    const int nfull = p.skv / 32;                    // blocks with 32 valid keys
-    for (int kbk = 0; kbk < nfull; ++kbk) key_block(kbk, unmasked{}, kbk == 0);
-    if (nfull < nkb) key_block(nfull, masked{}, nfull == 0);
-  }
+  const int nfull = p.skv / 32;                    // blocks with 32 valid keys
+  for (int kbk = 0; kbk < nfull; ++kbk) key_block(kbk, unmasked{}, kbk == 0);
+  if (nfull < nkb) key_block(nfull, masked{}, nfull == 0);
 
   // ---- O = (O^T / l)^T: lane holds query l%32, dh rows 8 (r/4) + 4 (l/32) + r%4 (+32 d) ----
 #pragma unroll
@@ -804,13 +767,13 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W == 4 ?
   }
 }
 
-template <int DH, int W>
 int32_t launch_res(AttnParams p, int skvp, hipStream_t st) {
+  constexpr int DH = 32, W = 8;
   p.q_tiles = static_cast<int>(cdiv(p.sq, W * 64));
   const int64_t blocks = static_cast<int64_t>(p.nb) * p.heads * p.q_tiles;
   if (blocks >= 0x7fffffffll) return set_error(WC_ERR_LIMIT, "wc_attention: too many tiles");
   const size_t lds = res_lds_bytes(DH, skvp);
-  auto kernel = p.causal ? attn_res_kernel<DH, W, true> : attn_res_kernel<DH, W, false>;
+  auto kernel = attn_res_kernel<DH, W>;
   if (lds > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
@@ -1212,16 +1175,25 @@ extern "C" int32_t wc_attention(const wc_attn_args* a, void* stream) {
   }
   p.dh = (int)a->head_dim;
   p.oc0 = 0;
-  if (al && !p.mask && a->dtype == WC_BF16 && (a->head_dim == 32 || a->head_dim == 64)) {
-    // resident-KV kernel: K and V of one head in LDS, 8-byte aligned output rows
+  if (al && !p.mask && !p.causal && a->dtype == WC_BF16 && a->head_dim == 32 && a->sq > 256) {
+    // resident-KV kernel: K and V of one head in LDS, 8-byte aligned output rows.  It folds the
+    // scale into Q and so needs one VALU instruction less per score than the streaming kernel,
+    // but stages all keys before it starts: worth it while its 512-query workgroups cover the
+    // CUs in one round or share a CU two at a time (128 x 8 heads of 512 tokens: 60.4 us against
+    // 69.4; 16 x 8 of 1000: 32.3 against 35.4; 16 x 8 of 512: 17.9 against 13.8; 64 x 8 of 700,
+    // four rounds of one workgroup per CU: 89 against 67)
     const int skvp = static_cast<int>(cdiv(a->skv, 32) * 32);
     const bool o_al = aligned(a->o, 8) && ubytes(a->o_stride_nb, es) % 8 == 0 && ubytes(a->o_stride_s, es) % 8 == 0;
-    if (o_al && res_lds_bytes((int)a->head_dim, skvp) <= 150 * 1024) {
-      const bool w8 = a->sq > 256;
-      if (a->head_dim == 32)
-        return w8 ? launch_res<32, 8>(p, skvp, as_stream(stream)) : launch_res<32, 4>(p, skvp, as_stream(stream));
-      return w8 ? launch_res<64, 8>(p, skvp, as_stream(stream)) : launch_res<64, 4>(p, skvp, as_stream(stream));
-    }
+    const size_t lds = res_lds_bytes(32, skvp);
+    const int64_t blocks = mul_sat({a->nb, a->heads, cdiv(a->sq, 512)});
+    const int cus = device_cu_count();
+    if (o_al && cus > 0 && lds <= 150 * 1024 && blocks >= cus && (blocks <= cus || lds <= 80 * 1024))
+      return launch_res(p, skvp, as_stream(stream));
+  }
+  if (al && a->dtype != WC_F32) {
+    const int32_t rc = a->dtype == WC_BF16 ? attn_stream<bf16>(p, as_stream(stream))
+                                           : attn_stream<f16>(p, as_stream(stream));
+    if (rc != 1) return rc;
   }
   if (a->dtype == WC_BF16) return launch_attn<bf16>(p, (int)a->head_dim, al, as_stream(stream));
   if (a->dtype == WC_F16) return launch_attn<f16>(p, (int)a->head_dim, al, as_stream(stream));

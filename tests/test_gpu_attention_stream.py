@@ -1,0 +1,110 @@
+"""The streaming 16-bit attention kernel (GPU) against fp64 and against the general kernel, which a
+mask of zeros selects: head dims on both sides of its padded widths, ragged numbers of queries
+and keys around its 32-key blocks and 64-key tiles, causal and full, cross lengths, non-finite
+values.
+
+Bar: P and the output are each rounded to the operand type (half an ulp, 2^-9 bf16 / 2^-12 fp16
+relative, on every value), Q K^T is exact products in fp32; the 2-norm error against fp64 stays
+under twice the sum of the two, and under 1.1 times the general kernel's."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+BAR = {torch.bfloat16: 4 * 2.0 ** -9, torch.float16: 4 * 2.0 ** -12}
+
+
+def _attend(q, k, v, heads, causal, masked):
+    """q [nb, sq, d], k / v [nb, skv, d] views with unit inner stride."""
+    from wide_compiler import _hip
+    nb, sq, d = q.shape
+    skv = k.shape[1]
+    o = torch.full((nb, sq, d), float("nan"), device=DEV, dtype=q.dtype)
+    mask = None
+    if masked:
+        mask = torch.zeros(1, 1, sq, skv, device=DEV)
+        if causal:
+            mask = mask.masked_fill(torch.ones(sq, skv, dtype=torch.bool, device=DEV).triu(1), float("-inf"))
+        mask = mask.expand(nb, heads, sq, skv)
+    _hip.attention(q=q, k=k, v=v, o=o, nb=nb, heads=heads, sq=sq, skv=skv, head_dim=d // heads,
+                   q_strides=q.stride()[:2], k_strides=k.stride()[:2], v_strides=v.stride()[:2],
+                   o_strides=(sq * d, d), scale=(d // heads) ** -0.5, causal=causal and not masked, mask=mask)
+    return o
+
+
+def _ref(q, k, v, heads, causal):
+    nb, sq, d = q.shape
+    skv = k.shape[1]
+    split = lambda t, s: t.double().reshape(nb, s, heads, d // heads).transpose(1, 2).contiguous()  # noqa: E731
+    a = split(q, sq) @ split(k, skv).transpose(2, 3).contiguous() * (d // heads) ** -0.5
+    if causal:
+        a = a.masked_fill(torch.ones(sq, skv, dtype=torch.bool, device=DEV).triu(1), float("-inf"))
+    return (torch.softmax(a, -1) @ split(v, skv)).transpose(1, 2).reshape(nb, sq, d)
+
+
+def _err(a, b):
+    return ((a.double() - b).norm() / b.norm()).item()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("nb,heads,dh,s", [
+    (3, 2, 8, 31), (2, 3, 16, 64), (1, 2, 24, 65), (2, 8, 32, 128), (4, 4, 32, 129), (1, 5, 40, 33),
+    (2, 2, 48, 257), (3, 2, 64, 1), (1, 1, 64, 63), (5, 8, 64, 96), (2, 8, 64, 300), (3, 1, 72, 127), (2, 2, 96, 66),
+    (1, 3, 120, 190), (2, 4, 128, 255), (64, 8, 64, 256), (32, 8, 32, 250), (40, 8, 96, 512)])
+def test_stream_attention(hip, nb, heads, dh, s, causal, dtype):
+    torch.manual_seed(nb * 1000 + dh + s)
+    d = heads * dh
+    qkv = torch.randn(nb, s, 3 * d, device=DEV).to(dtype)
+    q, k, v = qkv[..., :d], qkv[..., d:2 * d], qkv[..., 2 * d:]
+    ref = _ref(q, k, v, heads, causal)
+    got = _attend(q, k, v, heads, causal, False)
+    assert not torch.isnan(got).any()
+    e, general = _err(got, ref), _err(_attend(q, k, v, heads, causal, True), ref)
+    assert e <= BAR[dtype], (e, general)
+    assert e <= 1.1 * general + 2.0 ** -16, (e, general)
+
+
+@pytest.mark.parametrize("sq,skv,causal", [(1, 300, False), (37, 1000, False), (300, 37, False), (70, 200, True),
+                                           (200, 70, True), (130, 1, False)])
+def test_stream_cross_lengths(hip, sq, skv, causal):
+    torch.manual_seed(sq + skv)
+    heads, dh = 4, 64
+    q = torch.randn(3, sq, heads * dh, device=DEV).to(torch.bfloat16)
+    kv = torch.randn(3, skv, 2 * heads * dh, device=DEV).to(torch.bfloat16)
+    k, v = kv[..., :heads * dh], kv[..., heads * dh:]
+    ref = _ref(q, k, v, heads, causal)
+    got = _attend(q, k, v, heads, causal, False)
+    assert _err(got, ref) <= BAR[torch.bfloat16]
+
+
+def test_stream_growing_scores(hip):
+    """Scores that grow along the keys move the running maximum in every tile; large ones leave
+    one key with all the weight."""
+    torch.manual_seed(9)
+    heads, dh, s = 2, 64, 333
+    q = torch.randn(2, s, heads * dh, device=DEV)
+    k = torch.randn(2, s, heads * dh, device=DEV) * torch.linspace(0.1, 12, s, device=DEV)[None, :, None]
+    v = torch.randn(2, s, heads * dh, device=DEV)
+    q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
+    for causal in (False, True):
+        assert _err(_attend(q, k, v, heads, causal, False), _ref(q, k, v, heads, causal)) <= BAR[torch.bfloat16]
+
+
+def test_stream_non_finite_values(hip):
+    """A NaN or infinity in one key, query or value reaches the rows that attend to it, and no row of
+    another head or batch entry."""
+    torch.manual_seed(10)
+    heads, dh, s = 2, 48, 100
+    q, k, v = (torch.randn(4, s, heads * dh, device=DEV).to(torch.bfloat16) for _ in range(3))
+    clean = _attend(q, k, v, heads, False, False)
+    q[0, 5, 3] = float("nan")
+    k[1, 7, 50] = float("nan")
+    v[2, 99, 1] = float("inf")
+    got = _attend(q, k, v, heads, False, False)
+    nan = torch.isnan(got)
+    assert nan[0, 5, :dh].all() and not nan[0, :5].any() and not nan[0, 6:].any() and not nan[0, 5, dh:].any()
+    assert nan[1, :, dh:].all() and not nan[1, :, :dh].any()
+    assert torch.isinf(got[2, :, 1]).all() and torch.equal(got[2, :, 2:], clean[2, :, 2:])
+    assert torch.equal(got[3], clean[3])
