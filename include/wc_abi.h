@@ -221,8 +221,8 @@ typedef struct wc_rnn_args {
 int64_t wc_rnn_workspace_bytes(const wc_rnn_args* args);
 
 /* Byte offset in the workspace of the int32 status word of the partitioned plan, or
- * -1 when these sizes use another plan.  wc_rnn_input_projection zeroes
- * it; the recurrence sets it to 1 if a cross-workgroup wait timed out, in which
+ * -1 when these sizes use another plan.  wc_rnn_input_projection (fp32: wc_rnn_recurrence)
+ * zeroes it; the recurrence sets it to 1 if a cross-workgroup wait timed out, in which
  * case out / h_n / c_n are invalid. */
 int64_t wc_rnn_status_offset(const wc_rnn_args* args);
 
@@ -256,6 +256,10 @@ int32_t wc_rnn_input_projection(const wc_rnn_args* args, void* stream);
  *    state on-chip for all steps and exchange h_t through device-coherent memory; a
  *    cooperative launch per (compute units / (hidden/128)) units (ordinary launches
  *    under stream capture).
+ *  - Partitioned plan in fp32 (LSTM or GRU, hidden above 128 up to 384, a multiple of 32,
+ *    16-byte aligned w_hh / h0 / out, long enough sequences): hidden/16 or hidden/32
+ *    workgroups per unit, exchanging h_t through the output; cooperative launches.  A
+ *    captured stream takes the next form instead.
  *  - Otherwise one launch per step (an MFMA gate GEMM fused with the cell update;
  *    hidden % 32 == 0). */
 int32_t wc_rnn_recurrence(const wc_rnn_args* args, void* stream);

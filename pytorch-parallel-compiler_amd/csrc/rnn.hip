@@ -625,7 +625,8 @@ extern "C" int64_t wc_rnn_workspace_bytes(const wc_rnn_args* a) {
 
 extern "C" int64_t wc_rnn_status_offset(const wc_rnn_args* a) {
   if (!a || !rnn_sizes_fit(a)) return -1;
-  return part_plan(a) ? part_status_offset(a) : -1;
+  if (part_plan(a)) return part_status_offset(a);
+  return part32_plan(a) ? part32_status_offset(a) : -1;
 }
 
 extern "C" int32_t wc_rnn_set_spin_limit(int32_t polls) { return part_set_spin_limit(polls); }
@@ -747,6 +748,12 @@ extern "C" int32_t wc_rnn_recurrence(const wc_rnn_args* a, void* stream) {
   if (p.n == 0 || p.batch == 0 || p.steps == 0) return WC_OK;
   WC_REQUIRE(a->w_hh && a->out, WC_ERR_NULL, "wc_rnn_recurrence: null pointer");
   if (part_plan(a)) return part_recurrence(a, as_stream(stream));
+  if (part32_plan(a)) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(as_stream(stream), &cap) != hipSuccess)
+      return set_error(WC_ERR_ARG, "wc_rnn_recurrence: stream capture status unavailable");
+    if (cap == hipStreamCaptureStatusNone) return part32_recurrence(a, as_stream(stream));
+  }
   if (!rnn_plan(gates, p.hid, p)) {
     // W_hh of one model does not fit a workgroup's registers: one launch per step
     const int es = dtype_size(a->dtype);

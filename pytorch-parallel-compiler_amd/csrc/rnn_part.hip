@@ -761,17 +761,12 @@ int32_t launch_part(const wc_rnn_args* a, hipStream_t st) {
   p.xch = reinterpret_cast<uint32_t*>(ws + l.xch);
   p.sync = reinterpret_cast<int*>(ws + l.sync);
   p.status = a->status ? static_cast<int*>(a->status) : reinterpret_cast<int*>(ws + l.status);
-  p.spin_limit = g_spin_limit.load(std::memory_order_relaxed);
+  p.spin_limit = part_spin_limit();
   const size_t lds = part_lds_bytes<H>();
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(st, &cap) != hipSuccess)
     return set_error(WC_ERR_ARG, "wc_rnn_recurrence: stream capture status unavailable");
-  // WC_RNN_COOPERATIVE=0 makes the eager launch an ordinary one too, like the one under
-  // capture (rocprofv3 7.2 crashes at exit after a cooperative launch and writes no trace)
-  static const bool cooperative = [] {
-    const char* v = getenv("WC_RNN_COOPERATIVE");
-    return !(v && v[0] == '0' && v[1] == '\0');
-  }();
+  const bool cooperative = part_cooperative();
   const void* fn = reinterpret_cast<const void*>(part_kernel<H, T, CELL>);
   // units of (model, 16-row chunk), at most one workgroup per compute unit per launch
   const int total = static_cast<int>(part_units(a));
@@ -833,6 +828,18 @@ bool part_plan(const wc_rnn_args* a) {
   if (a->hidden == 384) return part_fits<384>(a);
   return part_fits<512>(a);
 }
+
+// WC_RNN_COOPERATIVE=0 makes eager launches ordinary ones, like those under capture (rocprofv3
+// 7.2 crashes at exit after a cooperative launch and writes no trace)
+bool part_cooperative() {
+  static const bool cooperative = [] {
+    const char* v = getenv("WC_RNN_COOPERATIVE");
+    return !(v && v[0] == '0' && v[1] == '\0');
+  }();
+  return cooperative;
+}
+
+int32_t part_spin_limit() { return g_spin_limit.load(std::memory_order_relaxed); }
 
 int64_t part_workspace_bytes(const wc_rnn_args* a) { return part_layout(a).total; }
 

@@ -32,5 +32,16 @@ int32_t part_set_spin_limit(int32_t polls);
 // receives its address (null when the layer has no bias)
 int32_t part_prepare(const wc_rnn_args* a, hipStream_t st, void** bias_f32);
 int32_t part_recurrence(const wc_rnn_args* a, hipStream_t st);
+// shared with the fp32 plan below: the current spin limit, and whether eager launches are
+// cooperative (the environment's WC_RNN_COOPERATIVE=0 makes them ordinary)
+int32_t part_spin_limit();
+bool part_cooperative();
+
+// ---- partitioned on-chip recurrence in fp32 (rnn_part32.hip) ----
+// true when it runs these sizes on the current device (outside stream capture); its counters live
+// in the workspace that the one-launch-per-step kernel sizes for its cell state
+bool part32_plan(const wc_rnn_args* a);
+int64_t part32_status_offset(const wc_rnn_args* a);
+int32_t part32_recurrence(const wc_rnn_args* a, hipStream_t st);
 
 }  // namespace wc

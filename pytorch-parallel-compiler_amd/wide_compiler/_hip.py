@@ -521,7 +521,10 @@ def rnn_set_spin_limit(polls: int) -> int:
 
 def _part_status(a: _RnnArgs, x: Tensor) -> Optional[Tensor]:
     """This device's status word, set in ``a``, when these sizes run the partitioned recurrence
-    (the one recurrent kernel with cross-workgroup waits); None otherwise."""
+    (the one recurrent kernel with cross-workgroup waits); None otherwise, and for a captured fp32
+    launch, which takes the kernel without such waits."""
+    if x.dtype == torch.float32 and torch.cuda.is_current_stream_capturing():
+        return None
     if int(lib().wc_rnn_status_offset(ctypes.byref(a))) < 0:
         return None
     word = rnn_status_word(x.device)

@@ -10,7 +10,8 @@ grouped MFMA GEMM for the input projection of all T steps, then one persistent r
 that keeps W_hh on-chip for all T steps (no per-step launches, no per-step HBM traffic for
 W_hh): for small hidden sizes each workgroup carries one (model, batch row) with its W_hh
 slice in registers; for bf16 / fp16 at hidden 256 / 384 / 512, hidden / 128 workgroups
-share a (model, 16-row chunk) and exchange h_t each step.  The launches are asynchronous; a
+share a (model, 16-row chunk) and exchange h_t each step, and so they do in fp32 for hidden
+sizes above 128 up to 384 (multiples of 32).  The launches are asynchronous; a
 bounded wait of the shared recurrence that gave up is raised by
 ``wide_compiler._hip.rnn_sync_check(block=True)`` or by the next recurrent call.
 """
