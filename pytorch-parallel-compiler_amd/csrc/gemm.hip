@@ -997,7 +997,7 @@ bool xl_shape_ok(const GemmParams& p) {
 //    (bf16 16 x 2048 x 128 x 1024: 19.0 against 29.8 with 128 x 128 tiles);
 //  - 128 x 128 tiles from two rounds of CUs on, unless the padding of short m or o wastes them
 //    (fp32 32 x 1024 x 256 x 256, 512 tiles: 34.4 against 37.7 with 64 x 64; 16 x 512 x 256 x 512,
-//    256 tiles: 22.6 against 21.9);
+//    256 tiles: 22.6 against 21.9) or, in fp32, k is short (64 x 400 x 16 x 512: 23.9 against 19.3);
 //  - 64 x 64 tiles while they cover the CUs (fp32 16 x 256 x 256 x 256, 256 tiles: 10.3 against
 //    11.7 with 32 x 32; 8 x 256 x 512 x 256, 128 tiles: 15.9 against 12.1).  Rows or columns that
 //    fill at most half of a 64-wide tile leave fp32 to the small tiles (64 x 16 x 256 x 1024:
@@ -1012,7 +1012,7 @@ int32_t launch_gemm_t(const GemmParams& p, bool vec, hipStream_t st) {
     if (vec && tiles(256) >= 256 && xl_shape_ok<TC>(p)) return launch_xl<TA, TB>(p, st);
   }
   const int64_t t128 = tiles(128), t64 = tiles(64), t32 = tiles(32);
-  if (t128 >= 512 && t128 * 7 <= t64 * 2) return gemm_tile<TA, TC, TB>(p, 128, st);
+  if (t128 >= 512 && t128 * 7 <= t64 * 2 && (sizeof(TA) == 2 || p.k >= 64)) return gemm_tile<TA, TC, TB>(p, 128, st);
   if (sizeof(TA) == 4 ? (t64 >= 192 && t32 * 2 > t64 * 5) : (t64 >= 256 || p.k > 64))
     return gemm_tile<TA, TC, TB>(p, 64, st);
   return launch_small<TA, TC, TB>(p, vec, st);

@@ -12,7 +12,7 @@
 // which holds every bit of a normal fp32 value (8 + 8 + 8 mantissa bits, round to nearest), and
 // the product is the sum of the six plane products of at most second order, accumulated in fp32.
 // The dropped terms are below 2^-26 of a product.  The bf16 MFMA does 16 times the fp32 one's
-// work per cycle, so six of them still take 2.7 times less, and each rounds the accumulator once
+// work per cycle, so six of them still take 2.7 times less, and each rounds its accumulator once
 // for 16 values of k: measured against fp64 the result is closer than the fp32 MFMA's.
 // Infinities and NaN (and values that round up to infinity in bf16) leave a NaN or an infinity
 // in the accumulator; a wave that finds one recomputes its tile with the fp32 MFMA from memory,
@@ -178,6 +178,15 @@ void gemm_tile_kernel(GemmParams p) {
     for (int j = 0; j < FN; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  // fp32, 64 x 64 tile: acc takes the largest plane product and low the five small ones, whose
+  // roundings are 2^-8 of acc's, so a k-step of 16 rounds the sum about once (2-norm error at k = 16
+  // 4.0e-8; 8.5e-8 with one accumulator, 7.8e-8 on the fp32 MFMA).  The 128 x 128 tile has no
+  // registers for it (it costs the third wave per SIMD and 8 %) and takes k >= 64 only, where one
+  // accumulator is closer than the fp32 MFMA too (1.35e-7 against 1.43e-7).
+  constexpr bool LOW = PLANES == 3 && FM * FN == 1;
+  f32x16 low;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) low[e] = 0.f;
 
   const int ksteps = (p.k + BK - 1) / BK;
   if (ksteps > 0) {
@@ -208,7 +217,10 @@ void gemm_tile_kernel(GemmParams p) {
 #pragma unroll
           for (int i = 0; i < FM; ++i)
 #pragma unroll
-            for (int j = 0; j < FN; ++j) acc[i][j] = mma32<TA>(wo[j][order - pa], am[i][pa], acc[i][j]);
+            for (int j = 0; j < FN; ++j) {
+              f32x16& c = LOW && order > 0 ? low : acc[i][j];
+              c = mma32<TA>(wo[j][order - pa], am[i][pa], c);
+            }
     }
     __syncthreads();
     if (kt + 1 < ksteps) {
@@ -218,6 +230,7 @@ void gemm_tile_kernel(GemmParams p) {
   }
 
   if constexpr (PLANES == 3) {
+    if constexpr (LOW) acc[0][0] += low;
     // infinities and NaN: the wave's tile again, with the fp32 MFMA straight from memory
     bool bad = false;
 #pragma unroll
