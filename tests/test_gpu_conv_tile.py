@@ -1,0 +1,114 @@
+"""The tile convolution kernel (GPU) against fp64: channel counts around its 16- and 32-channel
+steps and 64-channel tiles, ragged images, strides, dilations, depth, a fused residual, BatchNorm
+and ReLU, and in fp32 (computed as bf16 plane products) non-finite values.
+
+Bars (2-norm): fp32 sums of K products, 2^-23 sqrt(K); 16-bit results: half an ulp of the output
+(2^-9 bf16, 2^-12 fp16) on each value, doubled."""
+
+import pytest
+import torch
+import torch.nn as nn
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+OUT_BAR = {torch.float32: 0.0, torch.bfloat16: 2 ** -8, torch.float16: 2 ** -11}
+
+
+def _params(mod, dtype):
+    return mod.weight.detach().to(dtype).double(), mod.bias.detach().to(dtype).double()
+
+
+def _check(got, ref, k):
+    assert got.shape == ref.shape
+    assert not torch.isnan(got).any()
+    err = ((got.double() - ref).norm() / ref.norm()).item()
+    bar = 2.0 ** -23 * k ** 0.5 + OUT_BAR[got.dtype]
+    assert err <= bar, (err, bar)
+
+
+# n, b, ci, co, kernel, stride, padding, dilation, h, w
+SHAPES = [(2, 2, 1, 1, (3, 3), 1, 1, 1, 9, 11), (1, 3, 16, 33, (3, 3), 1, 1, 1, 16, 16), (3, 1, 17, 64, (1, 1), 1, 0, 1, 13, 10),
+          (2, 1, 31, 65, (3, 3), 2, 1, 1, 33, 35), (2, 2, 33, 40, (5, 5), 1, 2, 1, 12, 130), (1, 1, 64, 31, (3, 3), 1, 2, 2, 20, 20),
+          (2, 1, 40, 100, (7, 7), 2, 3, 1, 31, 29), (4, 2, 96, 64, (1, 3), 1, 0, 1, 1, 70), (1, 2, 48, 16, (3, 1), (2, 1), 1, 1, 40, 5),
+          (2, 1, 32, 32, (3, 3), 1, 1, 1, 1, 1), (1, 1, 8, 24, (4, 6), 3, 2, 1, 50, 64), (2, 1, 16, 16, (3, 3), 1, 0, 5, 30, 31)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,b,ci,co,kernel,stride,pad,dil,h,w", SHAPES)
+def test_conv_tile_shapes(hip, n, b, ci, co, kernel, stride, pad, dil, h, w, dtype):
+    import wide_compiler as wc
+    torch.manual_seed(ci * 100 + co)
+    mods = [nn.Conv2d(ci, co, kernel, stride=stride, padding=pad, dilation=dil) for _ in range(n)]
+    wide = wc.WideConv2d.from_modules(mods).to(DEV, dtype)
+    x = torch.randn(n, b, ci, h, w).to(dtype)
+    with torch.no_grad():
+        got = wide(x.to(DEV))
+        refs = []
+        for q, m in enumerate(mods):
+            wt, bias = _params(m, dtype)
+            refs.append(nn.functional.conv2d(x[q].double(), wt, bias, m.stride, m.padding, m.dilation))
+    _check(got.cpu(), torch.stack(refs), ci * kernel[0] * kernel[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_conv_tile_depth(hip, dtype):
+    import wide_compiler as wc
+    torch.manual_seed(1)
+    mods = [nn.Conv3d(20, 36, (3, 2, 3), stride=(2, 1, 1), padding=(1, 0, 1)) for _ in range(2)]
+    wide = wc.WideConv3d.from_modules(mods).to(DEV, dtype)
+    x = torch.randn(2, 2, 20, 7, 9, 14).to(dtype)
+    with torch.no_grad():
+        got = wide(x.to(DEV))
+        refs = []
+        for q, m in enumerate(mods):
+            wt, bias = _params(m, dtype)
+            refs.append(nn.functional.conv3d(x[q].double(), wt, bias, m.stride, m.padding))
+    _check(got.cpu(), torch.stack(refs), 20 * 18)
+
+
+@pytest.mark.parametrize("hw", [12, 13])
+def test_conv_tile_fused_epilogue(hip, hw):
+    """conv - BN - (+ residual) - ReLU in one launch, with 16-byte rows (12) and without (13)."""
+    from wide_compiler import _hip
+    torch.manual_seed(2)
+    n, b, ci, co = 3, 2, 24, 40
+    x, r = torch.randn(n, b, ci, hw, hw, device=DEV), torch.randn(n, b, co, hw, hw, device=DEV)
+    wt = torch.randn(n * co, ci, 3, 3, device=DEV) * 0.1
+    bias, g, be, mu = (torch.randn(n * co, device=DEV) for _ in range(4))
+    var = torch.rand(n * co, device=DEV) + 0.5
+    y = torch.full((n, b, co, hw, hw), float("nan"), device=DEV)
+    _hip.conv2d(x=x, weight=wt, n=n, c_in=ci, c_out=co, kernel=(3, 3), stride=(1, 1), padding=(1, 1),
+                dilation=(1, 1), y=y, bias=bias, bn=(g, be, mu, var, 1e-5), residual=r, relu=True)
+    refs = []
+    for q in range(n):
+        s = slice(q * co, (q + 1) * co)
+        v = nn.functional.conv2d(x[q].double().cpu(), wt[s].double().cpu(), bias[s].double().cpu(), padding=1)
+        a = [t[s].double().cpu()[None, :, None, None] for t in (mu, var, g, be)]
+        refs.append(torch.relu((v - a[0]) / (a[1] + 1e-5).sqrt() * a[2] + a[3] + r[q].double().cpu()))
+    _check(y.cpu(), torch.stack(refs), ci * 9)
+
+
+def test_conv_tile_fp32_special_values(hip):
+    """Infinities, NaN and values above the largest bf16 reach exactly the outputs that read them."""
+    import wide_compiler as wc
+    torch.manual_seed(3)
+    mods = [nn.Conv2d(20, 40, 3, padding=1) for _ in range(5)]
+    wide = wc.WideConv2d.from_modules(mods).to(DEV)
+    x = torch.randn(5, 2, 20, 17, 19)
+    x[0, 0, 3, 5, 6] = float("inf")
+    x[1, 1, 19, 16, 18] = float("nan")
+    x[2, 0, 0, 0, 0] = torch.finfo(torch.float32).max        # an infinity as a bf16
+    with torch.no_grad():
+        wide.grouped_conv.weight[3 * 40 + 7, 2, 1, 1] = -float("inf")
+        mods[3].weight[7, 2, 1, 1] = -float("inf")
+        got = wide(x.to(DEV)).cpu()
+        ref = torch.stack([nn.functional.conv2d(x[q].double(), m.weight.double(), m.bias.double(), padding=1)
+                           for q, m in enumerate(mods)])
+    f = ref.float()
+    assert torch.equal(torch.isnan(got), torch.isnan(f))
+    assert torch.equal(torch.isinf(got), torch.isinf(f))
+    assert torch.equal(torch.sign(got[torch.isinf(got)]), torch.sign(f[torch.isinf(f)]))
+    for q in range(5):
+        ok = torch.isfinite(f[q]) & (f[q].abs() < 1e30)
+        err = ((got[q][ok].double() - ref[q][ok]).norm() / ref[q][ok].norm()).item()
+        assert err <= 2.0 ** -23 * 180 ** 0.5
