@@ -5,8 +5,9 @@
 // layout the projection GEMMs produce (head h = columns [h*Dh, (h+1)*Dh)), so no
 // head-major copies are made.
 //
-// Three kernels here, next to the streaming 16-bit one (attention_stream.hip): attn_kernel, the
-// general one (fp32, masks, head dims and rows the others do not take), attn_res_kernel (bf16,
+// Three kernels here, next to the streaming ones (attention_stream.hip for 16-bit types,
+// attention_stream32.hip for fp32): attn_kernel, the general one (masks, head dims and rows the
+// others do not take), attn_res_kernel (bf16,
 // head dim 32, K and V resident in LDS) and attn_qkv_kernel (the same with the projections
 // inside).
 //
@@ -1190,9 +1191,10 @@ extern "C" int32_t wc_attention(const wc_attn_args* a, void* stream) {
     if (o_al && cus > 0 && lds <= 150 * 1024 && blocks >= cus && (blocks <= cus || lds <= 80 * 1024))
       return launch_res(p, skvp, as_stream(stream));
   }
-  if (al && a->dtype != WC_F32) {
-    const int32_t rc = a->dtype == WC_BF16 ? attn_stream<bf16>(p, as_stream(stream))
-                                           : attn_stream<f16>(p, as_stream(stream));
+  if (al) {
+    const int32_t rc = a->dtype == WC_F32    ? attn_stream32(p, as_stream(stream))
+                       : a->dtype == WC_BF16 ? attn_stream<bf16>(p, as_stream(stream))
+                                             : attn_stream<f16>(p, as_stream(stream));
     if (rc != 1) return rc;
   }
   if (a->dtype == WC_BF16) return launch_attn<bf16>(p, (int)a->head_dim, al, as_stream(stream));

@@ -34,7 +34,6 @@
 namespace wc {
 namespace {
 
-constexpr int kStBK = 64;              // keys per tile
 
 template <typename T>
 __device__ __forceinline__ f32x16 st_mma(bf16x8 a, bf16x8 b, f32x16 c) {
@@ -71,24 +70,6 @@ __device__ __forceinline__ float st_add2(uint32_t pair, float acc) {
   }
 }
 
-// DHP: the head dim rounded up to a multiple of 32 (columns past p.dh are zero in LDS).
-// Bank conflicts: K's 16-byte chunks are permuted within a row so that 16 rows' reads of one
-// chunk index cover the 64 banks; V's 64-byte blocks so that 4 consecutive rows' do.
-template <int DHP>
-__device__ __forceinline__ int k_at(int row, int c) {          // element offset of chunk c
-  if constexpr (DHP == 32) c ^= (row >> 1) & 3;
-  else if constexpr (DHP == 64) c ^= (row >> 1) & 7;
-  else if constexpr (DHP == 96) c ^= (row >> 2) & 3;
-  else c ^= row & 15;
-  return row * DHP + c * 8;
-}
-template <int DHP>
-__device__ __forceinline__ int v_at(int row, int col) {
-  if constexpr (DHP == 64) col ^= ((row >> 1) & 1) << 5;
-  else if constexpr (DHP == 128) col ^= (row & 3) << 5;
-  return row * DHP + col;
-}
-
 template <typename T, int DHP, int W, bool CAUSAL>
 __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(DHP <= 64 ? 4 : 2)))
 void attn_stream_kernel(AttnParams p) {
@@ -104,31 +85,8 @@ void attn_stream_kernel(AttnParams p) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int l32 = lane & 31, hf = lane >> 5;
 
-  // workgroup -> (head, query tile).  XCD x takes every head in [x, x + 1) * heads / 8, whose K
-  // and V then stay in its L2.  Causal tiles differ in length: the longest of all its heads come
-  // first, and every second round of one workgroup per CU runs backwards, so that a CU that
-  // started with a long tile goes on with a short one.
-  const int bhs = p.nb * p.heads;
   int bh, qt;
-  {
-    int heads = bhs, i = blockIdx.x, h0 = 0, cus = 256;
-    if ((bhs & 7) == 0) {
-      heads = bhs >> 3;
-      h0 = (blockIdx.x & 7) * heads;
-      i = blockIdx.x >> 3;
-      cus = 32;
-    }
-    if (CAUSAL) {
-      const int round = i / cus;
-      if ((round & 1) && (round + 1) * cus <= heads * p.q_tiles) i = round * cus + cus - 1 - (i - round * cus);
-      const int t = i / heads;
-      qt = p.q_tiles - 1 - t;
-      bh = h0 + i - t * heads;
-    } else {
-      bh = h0 + i / p.q_tiles;
-      qt = i % p.q_tiles;
-    }
-  }
+  stream_tile<CAUSAL>(p, bh, qt);
   const int nb = bh / p.heads, h = bh - (bh / p.heads) * p.heads;
   const int dh = p.dh;
   const T* qb = static_cast<const T*>(p.q) + nb * p.q_sb + static_cast<int64_t>(h) * dh;

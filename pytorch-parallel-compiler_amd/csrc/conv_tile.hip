@@ -49,22 +49,7 @@ __device__ __forceinline__ void ct_planes(const T (&v)[8], uint4 (&pl)[PLANES]) 
   if constexpr (PLANES == 1) {
     __builtin_memcpy(&pl[0], v, 16);
   } else {
-    float f[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) f[e] = v[e];
-#pragma unroll
-    for (int q = 0; q < PLANES; ++q) {
-      uint32_t h[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        h[e] = pack_bf16x2(f[2 * e], f[2 * e + 1]);
-        if (q < 2) {
-          f[2 * e] -= bf16_lo(h[e]);
-          f[2 * e + 1] -= bf16_hi(h[e]);
-        }
-      }
-      pl[q] = make_uint4(h[0], h[1], h[2], h[3]);
-    }
+    split_planes(v, pl);
   }
 }
 

@@ -57,14 +57,6 @@ template <> struct Unit<float> { uint4 v[2]; };
 template <> struct Unit<bf16> { uint4 v[1]; };
 template <> struct Unit<f16> { uint4 v[1]; };
 
-// two floats -> their bf16 parts in one dword, and what is left of them
-__device__ __forceinline__ uint32_t split_pair(float& lo, float& hi) {
-  const uint32_t h = pack_bf16x2(lo, hi);
-  lo -= bf16_lo(h);
-  hi -= bf16_hi(h);
-  return h;
-}
-
 template <typename TA, int FM, int FN>
 struct TileCfg {
   static constexpr int PLANES = sizeof(TA) == 4 ? 3 : 1;
@@ -158,14 +150,10 @@ void gemm_tile_kernel(GemmParams p) {
       } else {
         float f[8];
         __builtin_memcpy(f, &reg[q], sizeof(f));
+        uint4 pl[3];
+        split_planes(f, pl);
 #pragma unroll
-        for (int pl = 0; pl < PLANES; ++pl) {
-          uint32_t h[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            h[e] = pl < 2 ? split_pair(f[2 * e], f[2 * e + 1]) : pack_bf16x2(f[2 * e], f[2 * e + 1]);
-          *reinterpret_cast<uint4*>(lds_at(pl, r, su)) = make_uint4(h[0], h[1], h[2], h[3]);
-        }
+        for (int z = 0; z < 3; ++z) *reinterpret_cast<uint4*>(lds_at(z, r, su)) = pl[z];
       }
     }
   };

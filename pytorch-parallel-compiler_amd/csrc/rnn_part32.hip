@@ -47,7 +47,6 @@ constexpr int kSyncInts = 64;          // one 256-byte block per unit:
 constexpr int kSyncStatus = 31;        //   [0, 31): steps finished, per part; status (unit 0's)
 constexpr int kSyncXcc = 32;           //   [32, 64): XCD + 1, per part
 constexpr int kSc1 = 16;               // buffer-op cache policy: device scope
-constexpr float kPlaneMax = 3.38e38f;  // below the largest finite bf16: a larger value may round to infinity
 
 struct P32Params {
   int rows, chunks, unit0, units, steps, hid, parts, spin_limit;   // units: of this launch
@@ -70,29 +69,15 @@ __device__ __forceinline__ void sync_store(int* p, int v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// 8 floats as three bf16 planes; true when one of them is infinite or so large that its first
-// plane may be (NaN stays NaN in the planes)
+// 8 floats as planes; true when one is infinite or may round to it (NaN stays NaN in the planes)
 __device__ __forceinline__ bool split8(const float (&v)[8], bf16x8 (&pl)[3]) {
-  float f[8];
   bool bad = false;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    f[e] = v[e];
-    bad |= __builtin_fabsf(v[e]) > kPlaneMax;
-  }
+  for (int e = 0; e < 8; ++e) bad |= __builtin_fabsf(v[e]) > kPlaneMax;
+  uint4 u[3];
+  split_planes(v, u);
 #pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    uint32_t h[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      h[e] = pack_bf16x2(f[2 * e], f[2 * e + 1]);
-      if (q < 2) {
-        f[2 * e] -= bf16_lo(h[e]);
-        f[2 * e + 1] -= bf16_hi(h[e]);
-      }
-    }
-    pl[q] = __builtin_bit_cast(bf16x8, make_uint4(h[0], h[1], h[2], h[3]));
-  }
+  for (int q = 0; q < 3; ++q) pl[q] = __builtin_bit_cast(bf16x8, u[q]);
   return bad;
 }
 

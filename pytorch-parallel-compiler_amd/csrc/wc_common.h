@@ -108,6 +108,29 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
 
+// 8 floats as three bf16 planes, v = v0 + v1 + v2 with v0 = bf16(v), v1 = bf16(v - v0),
+// v2 = v - v0 - v1: every bit of a normal fp32 value above 2^-109.  Infinities, NaN and values
+// above kPlaneMax (they may round to infinity) leave NaN in the planes.
+constexpr float kPlaneMax = 3.38e38f;
+__device__ __forceinline__ void split_planes(const float (&v)[8], uint4 (&pl)[3]) {
+  float f[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) f[e] = v[e];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    uint32_t h[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      h[e] = pack_bf16x2(f[2 * e], f[2 * e + 1]);
+      if (q < 2) {
+        f[2 * e] -= __builtin_bit_cast(float, h[e] << 16);
+        f[2 * e + 1] -= __builtin_bit_cast(float, h[e] & 0xffff0000u);
+      }
+    }
+    pl[q] = make_uint4(h[0], h[1], h[2], h[3]);
+  }
+}
+
 // v_mfma_f32_16x16x32 on 16-bit operands carried as raw 16-byte fragments: the bf16 or
 // the fp16 instruction by the element type T
 template <typename T>
