@@ -707,14 +707,22 @@ __global__ void part_prep_kernel(int* sync, int64_t nsync, uint32_t* xch, int64_
   }
 }
 
+// Whether one workgroup fits a compute unit (and its LDS attribute set), found out once per device:
+// the plan is consulted several times per forward
 template <int H, typename T, int CELL>
 bool part_kernel_fits() {
+  static std::atomic<int> known[64];                 // per device: 0 unknown, 1 yes, 2 no
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
+  const int k = known[dev].load(std::memory_order_acquire);
+  if (k != 0) return k == 1;
   const size_t lds = part_lds_bytes<H>();
   const void* fn = reinterpret_cast<const void*>(part_kernel<H, T, CELL>);
-  if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) != hipSuccess)
-    return false;
   int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kPartThreads, lds) != hipSuccess) return false;
+  if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kPartThreads, lds) != hipSuccess)
+    return false;
+  known[dev].store(per_cu >= 1 ? 1 : 2, std::memory_order_release);
   return per_cu >= 1;
 }
 

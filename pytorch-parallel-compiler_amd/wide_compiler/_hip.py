@@ -18,6 +18,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 from typing import Dict, List, Optional, Sequence
 
 import torch
@@ -151,6 +152,20 @@ class _SelfAttnArgs(ctypes.Structure):
     ]
 
 
+def _packer(cls):
+    """struct.pack for the fields of an argument struct in order (pointers as integers, 0 for NULL):
+    the bytes of the C struct.  Packing a call's ~25 fields at once costs a third of setting them
+    one by one on a ctypes structure."""
+    codes = {ctypes.c_int32: "i", ctypes.c_int64: "q", ctypes.c_void_p: "P", ctypes.c_float: "f"}
+    s = struct.Struct("@" + "".join(codes[t] for _, t in cls._fields_) + "0q")
+    if s.size != ctypes.sizeof(cls):
+        raise ImportError(f"wide_compiler: {cls.__name__} packs to {s.size} bytes, not {ctypes.sizeof(cls)}")
+    return s.pack
+
+
+_pack_gemm, _pack_conv = _packer(_GemmArgs), _packer(_ConvArgs)
+_pack_attn, _pack_self_attn = _packer(_AttnArgs), _packer(_SelfAttnArgs)
+
 _P = ctypes.c_void_p
 _I32 = ctypes.c_int32
 _I64 = ctypes.c_int64
@@ -253,12 +268,39 @@ def stream_of(t: Tensor) -> int:
     """The current HIP stream of t's device as an address (what the ABI's void* stream takes).
     torch's raw accessor costs a tenth of building a torch.cuda.Stream object per launch."""
     if _raw_stream is not None:
-        return _raw_stream(t.device.index)
+        return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def ptr(t: Optional[Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
+
+
+try:
+    # CPython launcher of the entry points (built beside libwide_hip.so): a call through it
+    # costs a fraction of a ctypes call, which dominates a small forward's host time
+    from . import _wc_launch
+except ImportError:     # not built: the ctypes binding of the same entry points
+    _wc_launch = None
+_entries: Dict[str, int] = {}
+
+
+def entry_address(name: str) -> int:
+    """Address of libwide_hip.so's entry point `name` (looked up once)."""
+    a = _entries.get(name)
+    if a is None:
+        a = _entries[name] = ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value
+    return a
+
+
+def _launch(name: str, cls, block: bytes, stream: int) -> None:
+    """Call the entry point `name` with the packed argument struct `block` (of type cls)."""
+    if _wc_launch is not None:
+        rc = _wc_launch.callb(_entries.get(name) or entry_address(name), block, stream)
+    else:
+        rc = getattr(lib(), name)(ctypes.byref(cls.from_buffer_copy(block)), stream)
+    if rc:
+        _check(rc, name)
 
 
 # ---------------------------------------------------------------------------------------
@@ -307,9 +349,15 @@ def embedding_layernorm(weight: Tensor, ids: Tensor, gamma: Tensor, beta: Option
 
 def layernorm(x: Tensor, x_ms: int, x_rs: int, gamma: Tensor, beta: Optional[Tensor], y: Tensor,
               y_ms: int, y_rs: int, n: int, rows_per_model: int, dim: int, eps: float) -> None:
-    _check(lib().wc_layernorm(x.data_ptr(), x_ms, x_rs, gamma.data_ptr(), ptr(beta), y.data_ptr(), y_ms, y_rs,
-                              n, rows_per_model, dim, float(eps), dtype_code(x.dtype, "layernorm"),
-                              dtype_code(gamma.dtype, "layernorm"), stream_of(x)), "wc_layernorm")
+    args = (x.data_ptr(), x_ms, x_rs, gamma.data_ptr(), 0 if beta is None else beta.data_ptr(), y.data_ptr(), y_ms,
+            y_rs, n, rows_per_model, dim, float(eps), dtype_code(x.dtype, "layernorm"),
+            dtype_code(gamma.dtype, "layernorm"), stream_of(x))
+    if _wc_launch is not None:
+        rc = _wc_launch.layernorm(_entries.get("wc_layernorm") or entry_address("wc_layernorm"), *args)
+    else:
+        rc = lib().wc_layernorm(*args)
+    if rc:
+        _check(rc, "wc_layernorm")
 
 
 def bn_eval(x: Tensor, xsn: int, xsb: int, weight: Optional[Tensor], bias: Optional[Tensor],
@@ -337,18 +385,13 @@ def grouped_gemm(*, n: int, m: int, o: int, k: int,
                  bias: Optional[Tensor] = None, bias_sn: int = 0,
                  residual: Optional[Tensor] = None, r_sn: int = 0, r_so: int = 0, r_si: int = 0,
                  relu: bool = False) -> None:
-    g = _GemmArgs()
-    g.dtype = dtype_code(a.dtype, "grouped_gemm")
-    g.out_dtype = dtype_code(c.dtype, "grouped_gemm")
-    g.bias_dtype = dtype_code(bias.dtype, "grouped_gemm") if bias is not None else g.dtype
-    g.act = ACT_RELU if relu else ACT_NONE
-    g.n, g.m, g.o, g.k = n, m, o, k
-    g.a, g.a_stride_n, g.a_stride_outer, g.a_stride_inner, g.a_rows_inner = a.data_ptr(), a_sn, a_so, a_si, a_rows_inner
-    g.w, g.w_stride_n = w.data_ptr(), w_sn
-    g.bias, g.bias_stride_n = ptr(bias), bias_sn
-    g.residual, g.r_stride_n, g.r_stride_outer, g.r_stride_inner = ptr(residual), r_sn, r_so, r_si
-    g.c, g.c_stride_n, g.c_stride_outer, g.c_stride_inner, g.c_rows_inner = c.data_ptr(), c_sn, c_so, c_si, c_rows_inner
-    _check(lib().wc_grouped_gemm(ctypes.byref(g), stream_of(a)), "wc_grouped_gemm")
+    dt = dtype_code(a.dtype, "grouped_gemm")
+    _launch("wc_grouped_gemm", _GemmArgs, _pack_gemm(
+        dt, dtype_code(c.dtype, "grouped_gemm"), dt if bias is None else dtype_code(bias.dtype, "grouped_gemm"),
+        ACT_RELU if relu else ACT_NONE, n, m, o, k, a.data_ptr(), a_sn, a_so, a_si, a_rows_inner,
+        w.data_ptr(), w_sn, 0 if bias is None else bias.data_ptr(), bias_sn,
+        0 if residual is None else residual.data_ptr(), r_sn, r_so, r_si,
+        c.data_ptr(), c_sn, c_so, c_si, c_rows_inner), stream_of(a))
 
 
 def mlp2_supported(dtype: torch.dtype, in_features: int, hidden: int, out_features: int) -> bool:
@@ -372,23 +415,6 @@ def mlp2_args(*, n: int, m: int, in_features: int, hidden: int, out_features: in
     a.x, a.x_stride_n, a.x_stride_outer, a.x_stride_inner, a.x_rows_inner = x.data_ptr(), x_sn, x_so, x_si, x_rows_inner
     a.w1, a.b1, a.w2, a.b2 = w1.data_ptr(), ptr(b1), w2.data_ptr(), ptr(b2)
     a.y, a.y_stride_n, a.y_stride_outer, a.y_stride_inner, a.y_rows_inner = y.data_ptr(), y_sn, y_so, y_si, y_rows_inner
-    return a
-
-
-try:
-    # CPython launcher of the entry points (built beside libwide_hip.so): a call through it
-    # costs a fraction of a ctypes call, which dominates a small forward's host time
-    from . import _wc_launch
-except ImportError:     # not built: the ctypes binding of the same entry points
-    _wc_launch = None
-_entries: Dict[str, int] = {}
-
-
-def entry_address(name: str) -> int:
-    """Address of libwide_hip.so's entry point `name` (looked up once)."""
-    a = _entries.get(name)
-    if a is None:
-        a = _entries[name] = ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value
     return a
 
 
@@ -539,7 +565,12 @@ def rnn_forward(**kw) -> None:
     rnn_sync_check()
     a, ws = rnn_args(**kw)
     word = _part_status(a, kw["x"])
-    _check(lib().wc_rnn_forward(ctypes.byref(a), stream_of(kw["x"])), "wc_rnn_forward")
+    if _wc_launch is not None:
+        rc = _wc_launch.call2(_entries.get("wc_rnn_forward") or entry_address("wc_rnn_forward"), ctypes.addressof(a),
+                              stream_of(kw["x"]))
+    else:
+        rc = lib().wc_rnn_forward(ctypes.byref(a), stream_of(kw["x"]))
+    _check(rc, "wc_rnn_forward")
     if word is not None:
         _rnn_watch(word)
 
@@ -565,8 +596,13 @@ def rnn_phase(a: _RnnArgs, phase: str, like: Tensor) -> None:
 def conv_pack_weights(w: Tensor, n: int, c_out: int, c_in: int, kh: int, kw: int) -> Tensor:
     elems = int(lib().wc_conv_packed_weight_elems(n, c_out, c_in, kh, kw))
     out = torch.empty(max(elems, 8), dtype=w.dtype, device=w.device)
-    _check(lib().wc_conv_pack_weights(w.data_ptr(), n, c_out, c_in, kh, kw, dtype_code(w.dtype, "conv"),
-                                      out.data_ptr(), stream_of(w)), "wc_conv_pack_weights")
+    args = (w.data_ptr(), n, c_out, c_in, kh, kw, dtype_code(w.dtype, "conv"), out.data_ptr(), stream_of(w))
+    if _wc_launch is not None:
+        rc = _wc_launch.conv_pack(_entries.get("wc_conv_pack_weights") or entry_address("wc_conv_pack_weights"), *args)
+    else:
+        rc = lib().wc_conv_pack_weights(*args)
+    if rc:
+        _check(rc, "wc_conv_pack_weights")
     return out
 
 
@@ -578,31 +614,27 @@ def conv2d(*, x: Tensor, weight: Tensor, n: int, c_in: int, c_out: int, kernel, 
     running_var, eps) or None.  The filters go to the kernel as they are where the library
     reads that layout (wc_conv2d_direct_weights), else (or with ``packed``) through one
     packing pass."""
-    a = _ConvArgs()
-    a.dtype = dtype_code(x.dtype, "conv")
     params = [t for t in (bias, *(bn[:4] if bn else ())) if t is not None]
-    a.param_dtype = dtype_code(params[0].dtype, "conv") if params else a.dtype
-    a.act = ACT_RELU if relu else ACT_NONE
-    a.n, a.batch, a.c_in, a.c_out = n, x.shape[1], c_in, c_out
-    a.h, a.w = x.shape[3], x.shape[4]
-    a.kh, a.kw = kernel
-    a.stride_h, a.stride_w = stride
-    a.pad_h, a.pad_w = padding
-    a.dil_h, a.dil_w = dilation
-    a.h_out, a.w_out = y.shape[3], y.shape[4]
-    a.x, a.x_stride_n, a.x_stride_b = x.data_ptr(), x.stride(0), x.stride(1)
-    a.weight = weight.data_ptr()
-    a.bias = ptr(bias)
-    if bn is not None:
-        a.bn_weight, a.bn_bias, a.bn_mean, a.bn_var = ptr(bn[0]), ptr(bn[1]), ptr(bn[2]), ptr(bn[3])
-        a.bn_eps = float(bn[4])
-    if residual is not None:
-        a.residual, a.r_stride_n, a.r_stride_b = residual.data_ptr(), residual.stride(0), residual.stride(1)
-    a.y, a.y_stride_n, a.y_stride_b = y.data_ptr(), y.stride(0), y.stride(1)
-    if packed or not lib().wc_conv2d_direct_weights(ctypes.byref(a)):
-        packed = conv_pack_weights(weight, n, c_out, c_in, a.kh, a.kw)
-        a.packed_weight = packed.data_ptr()
-    _check(lib().wc_conv2d(ctypes.byref(a), stream_of(x)), "wc_conv2d")
+    dt = dtype_code(x.dtype, "conv")
+    bn_ptrs = (0, 0, 0, 0, 0.0) if bn is None else (ptr(bn[0]) or 0, ptr(bn[1]) or 0, ptr(bn[2]) or 0,
+                                                    ptr(bn[3]) or 0, float(bn[4]))
+    kh, kw = kernel
+    xs, ys = x.shape, y.shape
+    head = (dt, dtype_code(params[0].dtype, "conv") if params else dt, ACT_RELU if relu else ACT_NONE,
+            n, xs[1], c_in, c_out, xs[3], xs[4], kh, kw, *stride, *padding, *dilation, ys[3], ys[4],
+            x.data_ptr(), x.stride(0), x.stride(1))
+    tail = (0 if bias is None else bias.data_ptr(), *bn_ptrs,
+            *((0, 0, 0) if residual is None else (residual.data_ptr(), residual.stride(0), residual.stride(1))),
+            y.data_ptr(), y.stride(0), y.stride(1), weight.data_ptr())
+    a = None
+    if dt == BF16 and not packed:                # only bf16 filters are ever read in their own layout
+        a = _pack_conv(*head, 0, *tail)
+        if not lib().wc_conv2d_direct_weights(ctypes.byref(_ConvArgs.from_buffer_copy(a))):
+            a = None
+    if a is None:
+        packed_w = conv_pack_weights(weight, n, c_out, c_in, kh, kw)
+        a = _pack_conv(*head, packed_w.data_ptr(), *tail)
+    _launch("wc_conv2d", _ConvArgs, a, stream_of(x))
 
 
 def conv3d(*, x: Tensor, packed_w: Tensor, n: int, c_in: int, c_out: int, kernel, stride, padding, dilation,
@@ -632,23 +664,17 @@ def attention(*, q: Tensor, k: Tensor, v: Tensor, o: Tensor, nb: int, heads: int
     """q/k/v/o are base pointers (views) of [nb, S, heads*head_dim]-shaped data with the given
     (stride_nb, stride_s) element strides; ``mask`` is an additive fp32 [nb, heads, sq, skv]
     view with a unit key stride (other strides may be 0)."""
-    a = _AttnArgs()
-    a.dtype = dtype_code(q.dtype, "attention")
-    a.causal = 1 if causal else 0
-    a.nb, a.heads, a.sq, a.skv, a.head_dim = nb, heads, sq, skv, head_dim
-    a.scale = float(scale)
-    a.q, (a.q_stride_nb, a.q_stride_s) = q.data_ptr(), q_strides
-    a.k, (a.k_stride_nb, a.k_stride_s) = k.data_ptr(), k_strides
-    a.v, (a.v_stride_nb, a.v_stride_s) = v.data_ptr(), v_strides
-    a.o, (a.o_stride_nb, a.o_stride_s) = o.data_ptr(), o_strides
+    mask_fields = (0, 0, 0, 0)
     if mask is not None:
         if mask.dtype != torch.float32 or tuple(mask.shape) != (nb, heads, sq, skv) or \
                 (skv > 1 and mask.stride(3) != 1) or mask.device != q.device:
             raise ValueError("attention mask must be an fp32 [nb, heads, sq, skv] view with unit key stride "
                              "on the query's device")
-        a.mask = mask.data_ptr()
-        a.mask_stride_nb, a.mask_stride_head, a.mask_stride_q = mask.stride(0), mask.stride(1), mask.stride(2)
-    _check(lib().wc_attention(ctypes.byref(a), stream_of(q)), "wc_attention")
+        mask_fields = (mask.data_ptr(), mask.stride(0), mask.stride(1), mask.stride(2))
+    _launch("wc_attention", _AttnArgs, _pack_attn(
+        dtype_code(q.dtype, "attention"), 1 if causal else 0, nb, heads, sq, skv, head_dim, float(scale),
+        q.data_ptr(), *q_strides, k.data_ptr(), *k_strides, v.data_ptr(), *v_strides, o.data_ptr(), *o_strides,
+        *mask_fields), stream_of(q))
 
 
 def self_attention(*, x: Tensor, q_weight: Tensor, kv_weight: Tensor, q_bias: Optional[Tensor],
@@ -658,20 +684,13 @@ def self_attention(*, x: Tensor, q_weight: Tensor, kv_weight: Tensor, q_bias: Op
     contiguous rows, biases [N, D] / [N, 2D] or None, o [N, B, S, D] contiguous (the attention
     output before the output projection)."""
     n, b, s, d = x.shape
-    a = _SelfAttnArgs()
-    a.dtype = dtype_code(x.dtype, "self_attention")
-    a.causal = 1 if causal else 0
-    a.n, a.b, a.s, a.d_model, a.heads = n, b, s, d, heads
-    a.scale = float(scale)
-    a.x, a.x_stride_n, a.x_stride_b, a.x_stride_s = x.data_ptr(), x.stride(0), x.stride(1), x.stride(2)
-    a.q_weight, a.q_weight_stride_n = q_weight.data_ptr(), q_weight.stride(0)
-    a.kv_weight, a.kv_weight_stride_n = kv_weight.data_ptr(), kv_weight.stride(0)
-    if q_bias is not None:
-        a.q_bias, a.q_bias_stride_n = q_bias.data_ptr(), q_bias.stride(0)
-    if kv_bias is not None:
-        a.kv_bias, a.kv_bias_stride_n = kv_bias.data_ptr(), kv_bias.stride(0)
-    a.o, a.o_stride_nb, a.o_stride_s = o.data_ptr(), o.stride(1), o.stride(2)
-    _check(lib().wc_self_attention(ctypes.byref(a), stream_of(x)), "wc_self_attention")
+    _launch("wc_self_attention", _SelfAttnArgs, _pack_self_attn(
+        dtype_code(x.dtype, "self_attention"), 1 if causal else 0, n, b, s, d, heads, float(scale),
+        x.data_ptr(), x.stride(0), x.stride(1), x.stride(2), q_weight.data_ptr(), q_weight.stride(0),
+        kv_weight.data_ptr(), kv_weight.stride(0),
+        *((0, 0) if q_bias is None else (q_bias.data_ptr(), q_bias.stride(0))),
+        *((0, 0) if kv_bias is None else (kv_bias.data_ptr(), kv_bias.stride(0))),
+        o.data_ptr(), o.stride(1), o.stride(2)), stream_of(x))
 
 
 def exported_symbols() -> List[str]:

@@ -11,6 +11,7 @@ strided levels is consumed in place -- including the N-first view of a channel-p
 
 from __future__ import annotations
 
+import math
 from typing import NamedTuple, Optional, Sequence, Tuple
 
 from torch import Tensor
@@ -38,6 +39,10 @@ def _collapse(sizes: Sequence[int], strides: Sequence[int]) -> Tuple[Tuple[int, 
 
 def rows_of(x: Tensor) -> Optional[Rows]:
     """Two-level row addressing of x = [N, *batch, F] with unit stride on F, or None."""
+    if x.dim() >= 2 and x.is_contiguous():
+        n, f = x.shape[0], x.shape[-1]
+        m = x.numel() // (n * f) if n and f else math.prod(x.shape[1:-1])
+        return Rows(m * f, 0, f, m if m > 0 else 1, m)
     if x.dim() < 2 or (x.shape[-1] > 1 and x.stride(-1) != 1):
         return None
     batch = x.shape[1:-1]

@@ -102,10 +102,13 @@ class WideLinear(nn.Module):
         x, r = rows_or_contiguous(x)
         batch = tuple(x.shape[1:-1])
         if out is None:
-            out = torch.empty((self.n, *batch, self.out_features), dtype=x.dtype, device=x.device)
-        cr = rows_of(out)
-        if cr is None or tuple(out.shape) != (self.n, *batch, self.out_features):
-            raise RuntimeError(f"{what}: output view {list(out.shape)} is not addressable")
+            o, m = self.out_features, r.rows
+            out = torch.empty((self.n, *batch, o), dtype=x.dtype, device=x.device)
+            cr = (m * o, 0, o, m if m > 0 else 1)             # rows_of a contiguous tensor
+        else:
+            cr = rows_of(out)
+            if cr is None or tuple(out.shape) != (self.n, *batch, self.out_features):
+                raise RuntimeError(f"{what}: output view {list(out.shape)} is not addressable")
         if r.rows == 0 or self.out_features == 0:
             return out
         w = w if w.is_contiguous() else w.contiguous()
@@ -113,7 +116,7 @@ class WideLinear(nn.Module):
             n=self.n, m=r.rows, o=self.out_features, k=self.in_features,
             a=x, a_sn=r.stride_n, a_so=r.stride_outer, a_si=r.stride_inner, a_rows_inner=r.rows_inner,
             w=w, w_sn=self.out_features * self.in_features,
-            c=out, c_sn=cr.stride_n, c_so=cr.stride_outer, c_si=cr.stride_inner, c_rows_inner=cr.rows_inner,
+            c=out, c_sn=cr[0], c_so=cr[1], c_si=cr[2], c_rows_inner=cr[3],
             bias=b, bias_sn=self.out_features, relu=relu,
         )
         return out
