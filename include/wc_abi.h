@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define WC_ABI_VERSION 5
+#define WC_ABI_VERSION 6
 
 /* element types */
 enum {
@@ -306,6 +306,21 @@ typedef struct wc_gemm_args {
 } wc_gemm_args;
 
 int32_t wc_grouped_gemm(const wc_gemm_args* args, void* stream);
+
+/* wc_grouped_gemm whose output columns come from two weights: columns [0, o1) from g.w / g.bias (rows
+ * of o1 outputs per model), columns [o1, g.o) from w2 / bias2 (g.o - o1 outputs) -- the query
+ * and key|value projections of self-attention (wide_attention.py:199-209), which read one input
+ * and write one Q|K|V buffer.  g.bias and bias2 are both of g.bias_dtype. */
+typedef struct wc_gemm_pair_args {
+  wc_gemm_args g;
+  const void* w2;
+  int64_t w2_stride_n;
+  const void* bias2;
+  int64_t bias2_stride_n;
+  int64_t o1;
+} wc_gemm_pair_args;
+
+int32_t wc_grouped_gemm_pair(const wc_gemm_pair_args* args, void* stream);
 
 /*
  * Two chained WideLinear stages in one launch -- replaces, for a traced

@@ -68,7 +68,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmParams p) {
   const int wm = wave / WN, wn = wave - (wave / WN) * WN;
 
   const TA* abase = static_cast<const TA*>(p.a) + static_cast<int64_t>(mdl) * p.a_sn;
-  const TA* wbase = static_cast<const TA*>(p.w) + static_cast<int64_t>(mdl) * p.w_sn;
+  const TA* wbase = gemm_w<TA>(p, mdl, o0);
 
   // per-thread global row pointers of the chunks it stages (fixed over K)
   const TA* arow[A_PT];
@@ -200,7 +200,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmParams p) {
   }
 
   // ---- epilogue: bias, residual, activation, store ----
-  const TB* bias = p.bias ? static_cast<const TB*>(p.bias) + static_cast<int64_t>(mdl) * p.b_sn : nullptr;
+  const TB* bias = gemm_bias<TB>(p, mdl, o0);
   TC* cbase = static_cast<TC*>(p.c) + static_cast<int64_t>(mdl) * p.c_sn;
   const TC* rbase = p.r ? static_cast<const TC*>(p.r) + static_cast<int64_t>(mdl) * p.r_sn : nullptr;
 #pragma unroll
@@ -1005,16 +1005,42 @@ bool xl_shape_ok(const GemmParams& p) {
 //    they take 64 x 64 tiles from the first on (1 x 64 x 2048 x 64: 15.2 against 20.2) unless k
 //    is short (64 x 64 x 64 x 64: 4.4 against 3.8);
 //  - 32 x 32 tiles otherwise: the most workgroups in flight and the fewest dependent MFMAs.
+//
+// A pair (p.o1 > 0) runs as one launch of the kernel its joint sizes select when its split lies on a
+// tile of it, and as two when it does not or when a half would take the XL kernel by itself.  (fp32
+// 32 x 1024 x 256, 256 + 512 columns: the self-attention forward 174 -> 158 us, a forward of tiny
+// models 43 -> 35; besides the launch, 512 and 1024 tiles fill 1 and 2
+// rounds of the CUs' 768 places, 1536 exactly 2.)
 template <typename TA, typename TC, typename TB>
 int32_t launch_gemm_t(const GemmParams& p, bool vec, hipStream_t st) {
-  auto tiles = [&](int b) { return static_cast<int64_t>(p.n) * cdiv(p.m, b) * cdiv(p.o, b); };
-  if constexpr (sizeof(TA) == 2 && sizeof(TC) == 2) {
-    if (vec && tiles(256) >= 256 && xl_shape_ok<TC>(p)) return launch_xl<TA, TB>(p, st);
+  auto tiles = [&](const GemmParams& g, int b) { return static_cast<int64_t>(g.n) * cdiv(g.m, b) * cdiv(g.o, b); };
+  auto xl = [&](const GemmParams& g) {
+    if constexpr (sizeof(TA) == 2 && sizeof(TC) == 2) return vec && tiles(g, 256) >= 256 && xl_shape_ok<TC>(g);
+    return false;
+  };
+  const int64_t t128 = tiles(p, 128), t64 = tiles(p, 64), t32 = tiles(p, 32);
+  int tile = kSmallTile;
+  if (t128 >= 512 && t128 * 7 <= t64 * 2 && (sizeof(TA) == 2 || p.k >= 64)) tile = 128;
+  else if (sizeof(TA) == 4 ? (t64 >= 192 && t32 * 2 > t64 * 5) : (t64 >= 256 || p.k > 64)) tile = 64;
+  if (p.o1 > 0) {
+    GemmParams first = p, second = p;
+    first.o = p.o1;
+    first.o1 = second.o1 = 0;
+    second.o = p.o - p.o1;
+    second.w = p.w2;
+    second.w_sn = p.w2_sn;
+    second.bias = p.bias2;
+    second.b_sn = p.b2_sn;
+    second.c = static_cast<TC*>(p.c) + p.o1;
+    if (p.r) second.r = static_cast<const TC*>(p.r) + p.o1;
+    if (p.o1 % tile != 0 || xl(first) || xl(second)) {
+      const int32_t rc = launch_gemm_t<TA, TC, TB>(first, vec, st);
+      return rc ? rc : launch_gemm_t<TA, TC, TB>(second, vec, st);
+    }
+  } else if (xl(p)) {
+    if constexpr (sizeof(TA) == 2 && sizeof(TC) == 2) return launch_xl<TA, TB>(p, st);
   }
-  const int64_t t128 = tiles(128), t64 = tiles(64), t32 = tiles(32);
-  if (t128 >= 512 && t128 * 7 <= t64 * 2 && (sizeof(TA) == 2 || p.k >= 64)) return gemm_tile<TA, TC, TB>(p, 128, st);
-  if (sizeof(TA) == 4 ? (t64 >= 192 && t32 * 2 > t64 * 5) : (t64 >= 256 || p.k > 64))
-    return gemm_tile<TA, TC, TB>(p, 64, st);
+  if (tile != kSmallTile) return gemm_tile<TA, TC, TB>(p, tile, st);
   return launch_small<TA, TC, TB>(p, vec, st);
 }
 
@@ -1029,15 +1055,16 @@ int32_t grouped_gemm(const GemmParams& p0, int32_t dtype, int32_t out_dtype, int
   const bool vec = common_vec_bytes({reinterpret_cast<uintptr_t>(p.a), reinterpret_cast<uintptr_t>(p.w),
                                      ubytes(p.k, es), ubytes(p.a_sn, es),
                                      ubytes(p.a_so, es), ubytes(p.a_si, es),
-                                     ubytes(p.w_sn, es)}) >= 16;
+                                     ubytes(p.w_sn, es), reinterpret_cast<uintptr_t>(p.w2),
+                                     ubytes(p.w2_sn, es)}) >= 16;
   if (dtype == WC_F32) {
-    if (out_dtype != WC_F32 || (p.bias && bias_dtype != WC_F32))
+    if (out_dtype != WC_F32 || ((p.bias || p.bias2) && bias_dtype != WC_F32))
       return set_error(WC_ERR_DTYPE, "wc_grouped_gemm: f32 inputs need f32 output and bias");
     return launch_gemm_t<float, float, float>(p, vec, st);
   }
   if (dtype == WC_BF16) {
-    const bool bias_f32 = p.bias && bias_dtype == WC_F32;
-    if (p.bias && bias_dtype != WC_F32 && bias_dtype != WC_BF16)
+    const bool bias_f32 = (p.bias || p.bias2) && bias_dtype == WC_F32;
+    if ((p.bias || p.bias2) && bias_dtype != WC_F32 && bias_dtype != WC_BF16)
       return set_error(WC_ERR_DTYPE, "wc_grouped_gemm: bias dtype %s", dtype_name(bias_dtype));
     if (out_dtype == WC_BF16)
       return bias_f32 ? launch_gemm_t<bf16, bf16, float>(p, vec, st)
@@ -1048,8 +1075,8 @@ int32_t grouped_gemm(const GemmParams& p0, int32_t dtype, int32_t out_dtype, int
     return set_error(WC_ERR_DTYPE, "wc_grouped_gemm: output dtype %s", dtype_name(out_dtype));
   }
   if (dtype == WC_F16) {
-    const bool bias_f32 = p.bias && bias_dtype == WC_F32;
-    if (p.bias && bias_dtype != WC_F32 && bias_dtype != WC_F16)
+    const bool bias_f32 = (p.bias || p.bias2) && bias_dtype == WC_F32;
+    if ((p.bias || p.bias2) && bias_dtype != WC_F32 && bias_dtype != WC_F16)
       return set_error(WC_ERR_DTYPE, "wc_grouped_gemm: bias dtype %s", dtype_name(bias_dtype));
     if (out_dtype == WC_F16)
       return bias_f32 ? launch_gemm_t<f16, f16, float>(p, vec, st) : launch_gemm_t<f16, f16, f16>(p, vec, st);
@@ -1064,12 +1091,12 @@ int32_t grouped_gemm(const GemmParams& p0, int32_t dtype, int32_t out_dtype, int
 
 using namespace wc;
 
-extern "C" int32_t wc_grouped_gemm(const wc_gemm_args* g, void* stream) {
-  clear_error();
+// checks g and fills p; 1 when there is nothing to compute
+static int32_t gemm_params(const wc_gemm_args* g, GemmParams& p) {
   WC_REQUIRE(g != nullptr, WC_ERR_NULL, "wc_grouped_gemm: null args");
   WC_REQUIRE(g->n >= 0 && g->m >= 0 && g->o >= 0 && g->k >= 0, WC_ERR_SHAPE,
              "wc_grouped_gemm: negative size");
-  if (g->n == 0 || g->m == 0 || g->o == 0) return WC_OK;
+  if (g->n == 0 || g->m == 0 || g->o == 0) return 1;
   WC_REQUIRE(g->a && g->w && g->c, WC_ERR_NULL, "wc_grouped_gemm: null pointer");
   WC_REQUIRE(g->act == WC_ACT_NONE || g->act == WC_ACT_RELU, WC_ERR_ARG, "wc_grouped_gemm: bad act");
   WC_REQUIRE(g->m < 0x7fffffffll && g->o < 0x7fffffffll && g->k < 0x7fffffffll && g->n < 0x7fffffffll,
@@ -1080,7 +1107,6 @@ extern "C" int32_t wc_grouped_gemm(const wc_gemm_args* g, void* stream) {
              "wc_grouped_gemm: rows_inner too large");
   WC_REQUIRE(g->residual == nullptr || g->out_dtype == g->dtype || g->out_dtype == WC_F32,
              WC_ERR_DTYPE, "wc_grouped_gemm: residual dtype");
-  GemmParams p;
   p.n = (int)g->n;
   p.m = (int)g->m;
   p.o = (int)g->o;
@@ -1104,5 +1130,30 @@ extern "C" int32_t wc_grouped_gemm(const wc_gemm_args* g, void* stream) {
   p.c_so = g->c_stride_outer;
   p.c_si = g->c_stride_inner;
   p.c_ri = make_fastdiv(static_cast<uint32_t>(g->c_rows_inner));
+  return WC_OK;
+}
+
+extern "C" int32_t wc_grouped_gemm(const wc_gemm_args* g, void* stream) {
+  clear_error();
+  GemmParams p;
+  const int32_t rc = gemm_params(g, p);
+  if (rc) return rc == 1 ? WC_OK : rc;
   return grouped_gemm(p, g->dtype, g->out_dtype, g->bias_dtype, as_stream(stream));
+}
+
+extern "C" int32_t wc_grouped_gemm_pair(const wc_gemm_pair_args* a, void* stream) {
+  clear_error();
+  WC_REQUIRE(a != nullptr, WC_ERR_NULL, "wc_grouped_gemm: null args");
+  GemmParams p;
+  const int32_t rc = gemm_params(&a->g, p);
+  if (rc) return rc == 1 ? WC_OK : rc;
+  WC_REQUIRE(a->o1 > 0 && a->o1 < a->g.o, WC_ERR_SHAPE, "wc_grouped_gemm: pair split %lld outside 0 .. %lld",
+             (long long)a->o1, (long long)a->g.o);
+  WC_REQUIRE(a->w2, WC_ERR_NULL, "wc_grouped_gemm: null second weight");
+  p.o1 = (int)a->o1;
+  p.w2 = a->w2;
+  p.w2_sn = a->w2_stride_n;
+  p.bias2 = a->bias2;
+  p.b2_sn = a->bias2_stride_n;
+  return grouped_gemm(p, a->g.dtype, a->g.out_dtype, a->g.bias_dtype, as_stream(stream));
 }

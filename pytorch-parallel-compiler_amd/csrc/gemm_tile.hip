@@ -97,7 +97,7 @@ void gemm_tile_kernel(GemmParams p) {
   const int mw = (wave >> 1) * FM * 32, ow = (wave & 1) * FN * 32;   // the wave's corner of the tile
 
   const TA* const abase = static_cast<const TA*>(p.a) + static_cast<int64_t>(mdl) * p.a_sn;
-  const TA* const wbase = static_cast<const TA*>(p.w) + static_cast<int64_t>(mdl) * p.w_sn;
+  const TA* const wbase = gemm_w<TA>(p, mdl, o0);
   auto a_row = [&](int m) {
     m = m < p.m ? m : p.m - 1;                       // rows past the end repeat the last one (not stored)
     const uint32_t outer = fdiv(static_cast<uint32_t>(m), p.a_ri);
@@ -258,7 +258,7 @@ void gemm_tile_kernel(GemmParams p) {
 
   // ---- epilogue: 32-row strips through LDS (the last step's barrier has freed it), so that
   // stores and residual loads run along rows ----
-  const TB* bias = p.bias ? static_cast<const TB*>(p.bias) + static_cast<int64_t>(mdl) * p.b_sn : nullptr;
+  const TB* const bias = gemm_bias<TB>(p, mdl, o0);
   TC* const cbase = static_cast<TC*>(p.c) + static_cast<int64_t>(mdl) * p.c_sn;
   const TC* const rbase = p.r ? static_cast<const TC*>(p.r) + static_cast<int64_t>(mdl) * p.r_sn : nullptr;
   constexpr int EP = C::EPI_PITCH;

@@ -31,7 +31,29 @@ struct GemmParams {
   FastDiv fd_ks, fd_tpm, fd_tm;
   int32_t c_bytes, r_bytes;
   int vec_c;                   // tile kernel only: C and R rows take 16-byte accesses
+  // a second weight and bias for the columns from o1 on (0: none); o1 is a multiple of the
+  // launched tile, so a workgroup reads one of the two (tile and small-tile kernels)
+  int o1 = 0;
+  const void* w2 = nullptr;
+  int64_t w2_sn = 0;
+  const void* bias2 = nullptr;
+  int64_t b2_sn = 0;
 };
+
+// Row 0 and bias element 0 of the weight that output columns o0 .. belong to, such that both are
+// indexed by the output column.
+template <typename TA>
+__device__ __forceinline__ const TA* gemm_w(const GemmParams& p, int mdl, int o0) {
+  if (p.o1 > 0 && o0 >= p.o1)
+    return static_cast<const TA*>(p.w2) + static_cast<int64_t>(mdl) * p.w2_sn - static_cast<int64_t>(p.o1) * p.k;
+  return static_cast<const TA*>(p.w) + static_cast<int64_t>(mdl) * p.w_sn;
+}
+template <typename TB>
+__device__ __forceinline__ const TB* gemm_bias(const GemmParams& p, int mdl, int o0) {
+  if (p.o1 > 0 && o0 >= p.o1)
+    return p.bias2 ? static_cast<const TB*>(p.bias2) + static_cast<int64_t>(mdl) * p.b2_sn - p.o1 : nullptr;
+  return p.bias ? static_cast<const TB*>(p.bias) + static_cast<int64_t>(mdl) * p.b_sn : nullptr;
+}
 
 // The tile kernel (gemm_tile.hip), with 128 x 128 or 64 x 64 tiles (bm); any sizes, strides and
 // alignments.

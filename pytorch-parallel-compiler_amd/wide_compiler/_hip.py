@@ -24,7 +24,7 @@ from typing import Dict, List, Optional, Sequence
 import torch
 from torch import Tensor
 
-ABI_VERSION = 5
+ABI_VERSION = 6
 
 F32, BF16, F16 = 0, 1, 2
 ACT_NONE, ACT_RELU = 0, 1
@@ -73,6 +73,14 @@ class _GemmArgs(ctypes.Structure):
         ("c", ctypes.c_void_p),
         ("c_stride_n", ctypes.c_int64), ("c_stride_outer", ctypes.c_int64),
         ("c_stride_inner", ctypes.c_int64), ("c_rows_inner", ctypes.c_int64),
+    ]
+
+
+class _GemmPairArgs(ctypes.Structure):
+    _fields_ = [
+        *_GemmArgs._fields_,                     # the embedded wc_gemm_args
+        ("w2", ctypes.c_void_p), ("w2_stride_n", ctypes.c_int64),
+        ("bias2", ctypes.c_void_p), ("bias2_stride_n", ctypes.c_int64), ("o1", ctypes.c_int64),
     ]
 
 
@@ -163,7 +171,7 @@ def _packer(cls):
     return s.pack
 
 
-_pack_gemm, _pack_conv = _packer(_GemmArgs), _packer(_ConvArgs)
+_pack_gemm, _pack_gemm_pair, _pack_conv = _packer(_GemmArgs), _packer(_GemmPairArgs), _packer(_ConvArgs)
 _pack_attn, _pack_self_attn = _packer(_AttnArgs), _packer(_SelfAttnArgs)
 
 _P = ctypes.c_void_p
@@ -192,6 +200,7 @@ SIGNATURES = {
     "wc_rnn_input_projection": (_I32, [ctypes.POINTER(_RnnArgs), _P]),
     "wc_rnn_recurrence": (_I32, [ctypes.POINTER(_RnnArgs), _P]),
     "wc_grouped_gemm": (_I32, [ctypes.POINTER(_GemmArgs), _P]),
+    "wc_grouped_gemm_pair": (_I32, [ctypes.POINTER(_GemmPairArgs), _P]),
     "wc_mlp2_supported": (_I32, [_I32, _I64, _I64, _I64]),
     "wc_mlp2": (_I32, [ctypes.POINTER(_Mlp2Args), _P]),
     "wc_conv_pack_weights": (_I32, [_P, _I64, _I64, _I64, _I64, _I64, _I32, _P, _P]),
@@ -392,6 +401,22 @@ def grouped_gemm(*, n: int, m: int, o: int, k: int,
         w.data_ptr(), w_sn, 0 if bias is None else bias.data_ptr(), bias_sn,
         0 if residual is None else residual.data_ptr(), r_sn, r_so, r_si,
         c.data_ptr(), c_sn, c_so, c_si, c_rows_inner), stream_of(a))
+
+
+def grouped_gemm_pair(*, n: int, m: int, k: int, o1: int, o2: int, a: Tensor, a_sn: int, a_so: int, a_si: int,
+                      a_rows_inner: int, w1: Tensor, bias1: Optional[Tensor], w2: Tensor, bias2: Optional[Tensor],
+                      c: Tensor) -> None:
+    """Columns [0, o1) of c [n, m, o1 + o2] (contiguous) from w1 [n, o1, k] / bias1 [n, o1], the rest from
+    w2 [n, o2, k] / bias2 (wc_grouped_gemm_pair); weights contiguous and of a's dtype, biases
+    contiguous and of one dtype."""
+    dt = dtype_code(a.dtype, "grouped_gemm")
+    o = o1 + o2
+    bias = bias1 if bias1 is not None else bias2
+    _launch("wc_grouped_gemm_pair", _GemmPairArgs, _pack_gemm_pair(
+        dt, dt, dt if bias is None else dtype_code(bias.dtype, "grouped_gemm"), ACT_NONE, n, m, o, k, a.data_ptr(), a_sn, a_so, a_si, a_rows_inner,
+        w1.data_ptr(), o1 * k, 0 if bias1 is None else bias1.data_ptr(), o1, 0, 0, 0, 0,
+        c.data_ptr(), m * o, 0, o, max(m, 1), w2.data_ptr(), o2 * k, 0 if bias2 is None else bias2.data_ptr(), o2, o1),
+        stream_of(a))
 
 
 def mlp2_supported(dtype: torch.dtype, in_features: int, hidden: int, out_features: int) -> bool:
@@ -701,7 +726,7 @@ def exported_symbols() -> List[str]:
 # (compile_model=True) dynamo does not trace into the ctypes call and its stream handle,
 # but ends the compiled region there and runs the call as is, so inductor never generates
 # code for the hot path.
-for _name in ("pack_rows", "swap01", "embedding_gather", "layernorm", "bn_eval", "group_norm", "grouped_gemm",
+for _name in ("pack_rows", "swap01", "embedding_gather", "layernorm", "bn_eval", "group_norm", "grouped_gemm", "grouped_gemm_pair",
               "mlp2", "mlp2_args", "mlp2_launch", "embedding_layernorm", "rnn_forward", "rnn_forward_noalloc", "rnn_phase", "conv_pack_weights", "conv2d", "conv3d",
               "attention", "self_attention", "rnn_sync_check", "rnn_status_word", "rnn_set_spin_limit"):
     globals()[_name] = torch.compiler.disable(globals()[_name])

@@ -30,6 +30,7 @@ import torch
 from torch import Tensor, nn
 
 from ... import _hip
+from .._layout import rows_or_contiguous
 
 
 class AttentionStrategy(Enum):
@@ -100,7 +101,6 @@ class WideAttention(nn.Module):
                  out: Optional[Tensor] = None, col0: int = 0) -> Tensor:
         """[N, B, T, D] @ W[n]^T + b -> [N, B, T, o] via the grouped GEMM (x read in place), or into
         columns [col0, col0 + o) of ``out`` [N, B, T, C] when given."""
-        from .._layout import rows_or_contiguous
         x, r = rows_or_contiguous(x)
         m = r.rows
         if out is None:
@@ -167,12 +167,19 @@ class WideAttention(nn.Module):
                                 heads=hh, scale=dh ** -0.5, causal=is_causal)
             return self._project(attn, ow, d * d, self.out_bias, d, d)
         if query is key and key is value:
-            # self-attention: the Q and K|V GEMMs write columns [0, D) and [D, 3D) of one
+            # self-attention: one launch writes the Q (columns [0, D)) and K|V projections into one
             # [N, B, T, 3D] = Q | K | V buffer, which the attention kernel reads in place; the
             # parameters are read as they are on every call (no concatenated copy to go stale)
             qkv = torch.empty((n, b, tq, 3 * d), dtype=query.dtype, device=query.device)
-            self._project(query, qw, d * d, self.q_bias, d, d, out=qkv, col0=0)
-            self._project(query, kvw, 2 * d * d, kvb, 2 * d, 2 * d, out=qkv, col0=d)
+            qr, r = rows_or_contiguous(query)
+            c = lambda t: None if t is None else (t if t.is_contiguous() else t.contiguous())  # noqa: E731
+            if self.q_bias is not None and kvb is not None and self.q_bias.dtype != kvb.dtype:
+                self._project(query, qw, d * d, self.q_bias, d, d, out=qkv, col0=0)
+                self._project(query, kvw, 2 * d * d, kvb, 2 * d, 2 * d, out=qkv, col0=d)
+            else:
+                _hip.grouped_gemm_pair(n=n, m=r.rows, k=d, o1=d, o2=2 * d, a=qr, a_sn=r.stride_n,
+                                       a_so=r.stride_outer, a_si=r.stride_inner, a_rows_inner=r.rows_inner,
+                                       w1=qw, bias1=c(self.q_bias), w2=kvw, bias2=c(kvb), c=qkv)
             q, k_t, v_t = qkv, qkv[..., d:], qkv[..., 2 * d:]
             q_strides = k_strides = v_strides = (tq * 3 * d, 3 * d)
             attn = torch.empty((n, b, tq, d), dtype=query.dtype, device=query.device)

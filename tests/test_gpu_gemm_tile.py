@@ -119,3 +119,22 @@ def test_tile_gemm_fp32_range(hip, scale):
     x = torch.randn(130, 128, 48, device=DEV) * scale
     w = torch.randn(130, 128, 48, device=DEV)
     _check(_run(x, w, None), _ref(x, w, None), 48)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,m,k,o1,o2", [(40, 200, 96, 128, 256), (100, 65, 40, 64, 128), (3, 20, 64, 32, 64),
+                                         (2, 33, 48, 50, 100), (5, 1, 16, 96, 7), (64, 260, 64, 192, 384),
+                                         (32, 1024, 64, 256, 512)])
+def test_gemm_pair(hip, n, m, k, o1, o2, dtype):
+    """Two weights and one output: splits on a tile of every kernel and off them, with and without bias,
+    equal to two separate calls to the bar and to fp64."""
+    from wide_compiler import _hip
+    torch.manual_seed(n + m + o1)
+    x = torch.randn(n, m, k, device=DEV).to(dtype)
+    w1, w2 = torch.randn(n, o1, k, device=DEV).to(dtype), torch.randn(n, o2, k, device=DEV).to(dtype)
+    b1, b2 = torch.randn(n, o1, device=DEV).to(dtype), torch.randn(n, o2, device=DEV).to(dtype)
+    for p1, p2 in ((b1, b2), (None, None), (b1, None), (None, b2)):
+        c = torch.full((n, m, o1 + o2), float("nan"), device=DEV, dtype=dtype)
+        _hip.grouped_gemm_pair(n=n, m=m, k=k, o1=o1, o2=o2, a=x, a_sn=m * k, a_so=0, a_si=k, a_rows_inner=m,
+                               w1=w1, bias1=p1, w2=w2, bias2=p2, c=c)
+        _check(c, torch.cat([_ref(x, w1, p1), _ref(x, w2, p2)], -1), k)
