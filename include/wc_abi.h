@@ -356,6 +356,16 @@ int32_t wc_mlp2_supported(int32_t dtype, int64_t in_features, int64_t hidden, in
 
 int32_t wc_mlp2(const wc_mlp2_args* args, void* stream);
 
+/* The same for any widths, strides and alignments (fp32, bf16, fp16) whose 16 rows of x and h fit
+ * LDS (in + hidden up to about 2,500 in fp32, 5,000 in 16 bits; each at most 4096) and whose
+ * weights have at least 8 elements each.
+ * wc_mlp2_any_supported is 1 where that holds and one launch is also expected to be faster than
+ * two GEMMs. */
+int32_t wc_mlp2_any_supported(int32_t dtype, int64_t n, int64_t m, int64_t in_features, int64_t hidden,
+                              int64_t out_features);
+
+int32_t wc_mlp2_any(const wc_mlp2_args* args, void* stream);
+
 /*
  * Convolution weights packed for wc_conv2d: out[i, co, r, s, c] = w[i*c_out + co, c, r, s]
  * for c < c_in and 0 for c_in <= c < Ci32 (c_in rounded up to 32).  w is the grouped

@@ -85,6 +85,7 @@ class _GemmPairArgs(ctypes.Structure):
 
 
 class _Mlp2Args(ctypes.Structure):
+    entry = "wc_mlp2"                  # the entry point the block is for
     _fields_ = [
         ("dtype", ctypes.c_int32), ("act1", ctypes.c_int32), ("act2", ctypes.c_int32),
         ("n", ctypes.c_int64), ("m", ctypes.c_int64), ("in_features", ctypes.c_int64),
@@ -203,6 +204,8 @@ SIGNATURES = {
     "wc_grouped_gemm_pair": (_I32, [ctypes.POINTER(_GemmPairArgs), _P]),
     "wc_mlp2_supported": (_I32, [_I32, _I64, _I64, _I64]),
     "wc_mlp2": (_I32, [ctypes.POINTER(_Mlp2Args), _P]),
+    "wc_mlp2_any_supported": (_I32, [_I32, _I64, _I64, _I64, _I64, _I64]),
+    "wc_mlp2_any": (_I32, [ctypes.POINTER(_Mlp2Args), _P]),
     "wc_conv_pack_weights": (_I32, [_P, _I64, _I64, _I64, _I64, _I64, _I32, _P, _P]),
     "wc_conv_packed_weight_elems": (_I64, [_I64, _I64, _I64, _I64, _I64]),
     "wc_conv2d": (_I32, [ctypes.POINTER(_ConvArgs), _P]),
@@ -420,19 +423,31 @@ def grouped_gemm_pair(*, n: int, m: int, k: int, o1: int, o2: int, a: Tensor, a_
 
 
 def mlp2_supported(dtype: torch.dtype, in_features: int, hidden: int, out_features: int) -> bool:
-    if dtype not in (torch.float32, torch.bfloat16):
-        return False
-    return bool(lib().wc_mlp2_supported(dtype_code(dtype, "mlp2"), in_features, hidden, out_features))
+    """True when two chained layers of these widths run as one launch, at least for few rows."""
+    return mlp2_entry(dtype, 1, 1, in_features, hidden, out_features) is not None
+
+
+def mlp2_entry(dtype: torch.dtype, n: int, m: int, in_features: int, hidden: int, out_features: int) -> Optional[str]:
+    """The entry point that runs n models of m rows as one launch: wc_mlp2 for the widths it takes,
+    else wc_mlp2_any where one launch is faster than two GEMMs; None: two GEMMs."""
+    if dtype not in _DTYPES:
+        return None
+    code = dtype_code(dtype, "mlp2")
+    if lib().wc_mlp2_supported(code, in_features, hidden, out_features):
+        return "wc_mlp2"
+    return "wc_mlp2_any" if lib().wc_mlp2_any_supported(code, n, m, in_features, hidden, out_features) else None
 
 
 def mlp2_args(*, n: int, m: int, in_features: int, hidden: int, out_features: int,
               x: Tensor, x_sn: int, x_so: int, x_si: int, x_rows_inner: int,
               w1: Tensor, b1: Optional[Tensor], w2: Tensor, b2: Optional[Tensor],
               y: Tensor, y_sn: int, y_so: int, y_si: int, y_rows_inner: int,
-              relu1: bool, relu2: bool) -> "_Mlp2Args":
-    """The filled argument block of wc_mlp2 (launch with mlp2_launch; a caller may keep it and
-    change only the x / y addresses between launches)."""
+              relu1: bool, relu2: bool, entry: str = "wc_mlp2") -> "_Mlp2Args":
+    """The filled argument block of wc_mlp2 or wc_mlp2_any (launch with mlp2_launch; a caller may
+    keep it and change only the x / y addresses between launches)."""
     a = _Mlp2Args()
+    if entry != a.entry:
+        a.entry = entry
     a.dtype = dtype_code(x.dtype, "mlp2")
     a.act1 = ACT_RELU if relu1 else ACT_NONE
     a.act2 = ACT_RELU if relu2 else ACT_NONE
@@ -444,12 +459,13 @@ def mlp2_args(*, n: int, m: int, in_features: int, hidden: int, out_features: in
 
 
 def mlp2_launch(a: "_Mlp2Args", stream: int) -> None:
+    name = a.entry
     if _wc_launch is not None:
-        rc = _wc_launch.call2(_entries.get("wc_mlp2") or entry_address("wc_mlp2"), ctypes.addressof(a), stream)
+        rc = _wc_launch.call2(_entries.get(name) or entry_address(name), ctypes.addressof(a), stream)
     else:
-        rc = lib().wc_mlp2(ctypes.byref(a), stream)
+        rc = getattr(lib(), name)(ctypes.byref(a), stream)
     if rc:
-        _check(rc, "wc_mlp2")
+        _check(rc, name)
 
 
 def mlp2(**kw) -> None:
@@ -727,7 +743,7 @@ def exported_symbols() -> List[str]:
 # but ends the compiled region there and runs the call as is, so inductor never generates
 # code for the hot path.
 for _name in ("pack_rows", "swap01", "embedding_gather", "layernorm", "bn_eval", "group_norm", "grouped_gemm", "grouped_gemm_pair",
-              "mlp2", "mlp2_args", "mlp2_launch", "embedding_layernorm", "rnn_forward", "rnn_forward_noalloc", "rnn_phase", "conv_pack_weights", "conv2d", "conv3d",
+              "mlp2", "mlp2_entry", "mlp2_args", "mlp2_launch", "embedding_layernorm", "rnn_forward", "rnn_forward_noalloc", "rnn_phase", "conv_pack_weights", "conv2d", "conv3d",
               "attention", "self_attention", "rnn_sync_check", "rnn_status_word", "rnn_set_spin_limit"):
     globals()[_name] = torch.compiler.disable(globals()[_name])
 del _name

@@ -142,8 +142,8 @@ class WideLinear(nn.Module):
 
 
 class WideMLP2(nn.Module):
-    """Two chained WideLinear stages (the first optionally followed by ReLU) run as one
-    wc_mlp2 launch; TracedWideModel builds it when it finds a Linear -> [ReLU] -> Linear
+    """Two chained WideLinear stages (the first optionally followed by ReLU) run as one launch
+    (wc_mlp2 or wc_mlp2_any; two GEMMs for more rows than that pays for); TracedWideModel builds it when it finds a Linear -> [ReLU] -> Linear
     chain whose intermediate has no other consumer.  The hidden activations never reach
     memory; they are rounded to the parameter dtype as the first stage would store them.
     Parameters stay in the two WideLinear modules (state_dict keys unchanged)."""
@@ -172,6 +172,19 @@ class WideMLP2(nn.Module):
     def _params(self):
         p1, p2 = self.first._parameters, self.second._parameters
         return p1["weight"], p1.get("bias"), p2["weight"], p2.get("bias")
+
+    def _entry(self, x: Tensor) -> Optional[str]:
+        """The entry point that runs x ([N, ..., in]) as one launch; None: two GEMMs."""
+        return _hip.mlp2_entry(self.first.weight.dtype, self.n, max(math.prod(x.shape[1:-1]), 1), self.in_features,
+                               self.hidden, self.out_features)
+
+    def split(self, x: Tensor) -> Optional[Tensor]:
+        """Where x is to run as two GEMMs, the first one's output; else None (nothing run).  A caller
+        that allocates the output can so do it after the hidden activations, as for two stages."""
+        plan = self.__dict__.get("_plan")
+        if (plan is not None and plan[0][0] == x.shape) or self._entry(x) is not None:
+            return None
+        return self.first.forward_into(x, None, relu=self.relu1)
 
     def plan_key(self, x: Tensor, out: Optional[Tensor], relu: bool, params) -> tuple:
         return (x.shape, x.stride(), x.dtype, x.device, None if out is None else (out.shape, out.stride()),
@@ -216,6 +229,9 @@ class WideMLP2(nn.Module):
         what = "WideMLP2"
         if x.dim() < 2 or x.shape[0] != self.n or x.shape[-1] != self.in_features:
             raise RuntimeError(f"{what}: expected input [N={self.n}, ..., {self.in_features}], got {list(x.shape)}")
+        entry = self._entry(x)
+        if entry is None:                                     # too many rows for one launch to pay
+            return self.second.forward_into(self.first.forward_into(x, None, relu=self.relu1), out, relu=relu)
         key_x, key_out = x, out
         _hip.require_device(what, x, *params)
         _hip.require_forward_only(what, x, *params)
@@ -238,7 +254,7 @@ class WideMLP2(nn.Module):
                               x=x, x_sn=r.stride_n, x_so=r.stride_outer, x_si=r.stride_inner,
                               x_rows_inner=r.rows_inner, w1=w1, b1=b1, w2=w2, b2=b2,
                               y=out, y_sn=cr.stride_n, y_so=cr.stride_outer, y_si=cr.stride_inner,
-                              y_rows_inner=cr.rows_inner, relu1=self.relu1, relu2=relu)
+                              y_rows_inner=cr.rows_inner, relu1=self.relu1, relu2=relu, entry=entry)
         _hip.mlp2_launch(args, _hip.stream_of(x))
         # keep the arguments for calls of the same form: x read in place (no copy made), the
         # parameters contiguous (their addresses are in the key), the output allocated here

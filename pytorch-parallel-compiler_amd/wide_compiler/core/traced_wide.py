@@ -596,6 +596,10 @@ class TracedWideModel(nn.Module):
     def _into_packed(self, op: nn.Module, x: Tensor, kwargs: Dict[str, Any]) -> Optional[Tuple[Tensor, Tensor]]:
         """Run the output stage writing straight into the packed [B, N*C, *S] layout when it
         is a WideLinear or WideConv2d; returns (packed, N-first view of it) or None."""
+        if isinstance(op, WideMLP2) and not kwargs and x.dim() >= 3:
+            hidden = op.split(x)
+            if hidden is not None:
+                x, op = hidden, op.second
         if isinstance(op, (WideLinear, WideMLP2)) and not kwargs and x.dim() >= 3:
             nf_shape = (x.shape[0], x.shape[1], *x.shape[2:-1], op.out_features)
         elif isinstance(op, WideConv2d) and set(kwargs) <= {"residual"} and x.dim() == 5:
