@@ -269,10 +269,12 @@ void conv_tile_kernel(ConvParams p) {
         for (int r = 0; r < p.kh; ++r)
           for (int s = 0; s < p.kw; ++s) {
             const int di = od * p.sd - p.pd + t * p.dd, hi = hi0 + pr * p.sh + r * p.dh, wi = wi0 + pc * p.sw + s * p.dw;
-            if (di < 0 || di >= p.d || hi < 0 || hi >= p.h || wi < 0 || wi >= p.w) continue;
-            const T* xp = xb + (static_cast<int64_t>(di) * p.h + hi) * p.w + wi;
+            if (di < 0 || di >= p.d) continue;
+            // a padding pixel is a zero that meets the weight: an infinite weight gives NaN there
+            const bool in = hi >= 0 && hi < p.h && wi >= 0 && wi < p.w;
+            const T* xp = xb + (static_cast<int64_t>(di) * p.h + (in ? hi : 0)) * p.w + (in ? wi : 0);
             const T* wp = wr + static_cast<int64_t>((t * p.kh + r) * p.kw + s) * p.ci32;
-            for (int c = 0; c < p.ci; ++c) v += to_f32(xp[c * p.x_cs]) * to_f32(wp[c]);
+            for (int c = 0; c < p.ci; ++c) v += (in ? to_f32(xp[c * p.x_cs]) : 0.f) * to_f32(wp[c]);
           }
       cs[(cw + l32) * CPITCH + px] = from_f32<T>(v * alpha + beta);
     }

@@ -112,3 +112,25 @@ def test_conv_tile_fp32_special_values(hip):
         ok = torch.isfinite(f[q]) & (f[q].abs() < 1e30)
         err = ((got[q][ok].double() - ref[q][ok]).norm() / ref[q][ok].norm()).item()
         assert err <= 2.0 ** -23 * 180 ** 0.5
+
+
+def test_conv_tile_fp32_infinite_weight_meets_padding(hip):
+    """A padding pixel is a zero like any other: times an infinite weight it is NaN, so the border
+    outputs whose window holds that tap over the padding are NaN and the others infinite."""
+    import wide_compiler as wc
+    torch.manual_seed(4)
+    mods = [nn.Conv2d(20, 40, 3, padding=1) for _ in range(2)]
+    x = torch.randn(2, 2, 20, 17, 19)
+    with torch.no_grad():
+        mods[1].weight[7, 2, 0, 0] = float("inf")
+        wide = wc.WideConv2d.from_modules(mods).to(DEV)
+        got = wide(x.to(DEV)).cpu()
+        refs = []
+        for q, m in enumerate(mods):
+            cols = nn.functional.unfold(x[q].double(), 3, padding=1)
+            ref = (m.weight.double().flatten(1) @ cols + m.bias.double()[:, None]).view(2, 40, 17, 19)
+            refs.append(ref)
+    f = torch.stack(refs).float()
+    assert torch.isnan(f[1, :, 7, 0]).all() and torch.isinf(f[1, :, 7, 1:, 1:]).all()
+    assert torch.equal(torch.isnan(got), torch.isnan(f))
+    assert torch.equal(torch.isinf(got), torch.isinf(f))
