@@ -421,8 +421,9 @@ int32_t wc_conv2d(const wc_conv_args* args, void* stream);
  * wide_conv2d.py:169-194), which reads grouped_conv.weight on every call: 1 when wc_conv2d
  * runs these sizes from args->weight directly (packed_weight NULL) -- the resident-weight
  * kernel (bf16 'same' convolution, stride 1, C_in 32 or 64, C_out a multiple of 64, the
- * input widths it is built for) stages the module's filter bank in its own layout, so no
- * packing pass precedes it; 0 otherwise (wc_conv_pack_weights, then wc_conv2d). */
+ * input widths it is built for) and, for few output tiles and at most 160 values per output
+ * channel, the tile kernel stage the module's filter bank in its own layout, so no packing pass
+ * precedes them (element alignment suffices for the tile kernel); 0 otherwise (wc_conv_pack_weights, then wc_conv2d). */
 int32_t wc_conv2d_direct_weights(const wc_conv_args* args);
 
 /*

@@ -924,7 +924,7 @@ extern "C" int64_t wc_conv_packed_weight_elems(int64_t n, int64_t c_out, int64_t
 }
 
 extern "C" int32_t wc_conv2d_direct_weights(const wc_conv_args* a) {
-  if (!a || a->dtype != WC_BF16 || !a->weight || a->n <= 0 || a->batch <= 0 || a->c_out <= 0 || a->h <= 0 ||
+  if (!a || dtype_size(a->dtype) == 0 || !a->weight || a->n <= 0 || a->batch <= 0 || a->c_out <= 0 || a->h <= 0 ||
       a->w <= 0 || a->stride_h <= 0 || a->stride_w <= 0 || a->dil_h <= 0 || a->dil_w <= 0)
     return 0;
   if (!fits_i32({a->n, a->batch, a->c_in, a->c_out, a->h, a->w, a->kh, a->kw, a->stride_h, a->stride_w,
@@ -932,6 +932,9 @@ extern "C" int32_t wc_conv2d_direct_weights(const wc_conv_args* a) {
       mul_sat({a->c_in, a->h, a->w}) >= 0x7fffffffll || mul_sat({a->n, a->c_out}) >= 0x7fffffffll)
     return 0;
   ConvParams p = {};
+  p.n = (int)a->n;
+  p.batch = (int)a->batch;
+  p.kd = p.sd = p.dd = p.d = p.dout = 1;
   p.ci = (int)a->c_in;
   p.co = (int)a->c_out;
   p.h = (int)a->h;
@@ -956,7 +959,10 @@ extern "C" int32_t wc_conv2d_direct_weights(const wc_conv_args* a) {
   p.y = a->y;
   p.y_sn = a->y_stride_n;
   p.y_sb = a->y_stride_b;
-  return conv_res_ok(p) ? 1 : 0;
+  if (a->dtype == WC_BF16 && conv_res_ok(p)) return 1;
+  return p.ci > 0 && p.kh > 0 && p.kw > 0 && p.ho > 0 && p.wo > 0 && p.ph >= 0 && p.pw >= 0 &&
+                 mul_sat({p.kh, p.kw, p.ci}) <= 160 && aligned(a->weight, dtype_size(a->dtype)) && conv_tile_raw(p, a->dtype)
+             ? 1 : 0;
 }
 
 extern "C" int32_t wc_conv2d(const wc_conv_args* a, void* stream) {
@@ -1039,11 +1045,12 @@ extern "C" int32_t wc_conv2d(const wc_conv_args* a, void* stream) {
   const bool ral = !p.res || (aligned(p.res, 16) && ubytes(p.r_sn, es) % 16 == 0 && ubytes(p.r_sb, es) % 16 == 0);
   p.vec_out = (yal && ral && p.tc % ve == 0 && p.wo % ve == 0) ? 1 : 0;
   if (p.wn) {
-    // the filter bank itself: only the resident-weight kernel reads that layout
-    WC_REQUIRE(!f32 && !f16m && conv_res_ok(p), WC_ERR_ARG,
+    // the filter bank itself: the resident-weight kernel, or the tile kernel on few tiles
+    const bool res = !f32 && !f16m && conv_res_ok(p);
+    WC_REQUIRE(res || (mul_sat({p.kh, p.kw, p.ci}) <= 160 && aligned(p.wn, es) && conv_tile_raw(p, a->dtype)), WC_ERR_ARG,
                "wc_conv2d: these sizes need packed weights (wc_conv_pack_weights); "
                "wc_conv2d_direct_weights tells when the filter bank itself will do");
-    return conv_res_dispatch(p, as_stream(stream));
+    return res ? conv_res_dispatch(p, as_stream(stream)) : conv_tile(p, a->dtype, "wc_conv2d", as_stream(stream));
   }
   WC_REQUIRE(aligned(p.wp, 16), WC_ERR_ALIGN, "wc_conv2d: packed weights not 16-byte aligned");
   const int64_t nblk = static_cast<int64_t>(p.n) * p.batch * p.tiles_r * p.tiles_c * p.tiles_co;

@@ -34,6 +34,13 @@ namespace {
 constexpr int kTPix = 128;             // output pixels per tile
 constexpr int kXPitch = 40;            // 16-bit elements per staged pixel (32 channels + 8)
 
+// elements per raw weight row: up to 32 channels of all taps, and 16 bytes against bank conflicts
+template <typename T>
+__host__ __device__ inline int raw_pitch(const ConvParams& p) {
+  constexpr int CE = 16 / sizeof(T);
+  return ((p.ci < 32 ? p.ci : 32) * p.kh * p.kw + CE - 1) / CE * CE + CE;
+}
+
 template <typename T>
 __device__ __forceinline__ f32x16 ct_mma(bf16x8 a, bf16x8 b, f32x16 c) {
   if constexpr (std::is_same<T, f16>::value)
@@ -53,7 +60,10 @@ __device__ __forceinline__ void ct_planes(const T (&v)[8], uint4 (&pl)[PLANES]) 
   }
 }
 
-template <typename T>
+// RAW: the weights come from the module's filter bank [co][ci][taps] instead of the packed layout.  A
+// 32-channel chunk's rows of all taps, contiguous per output channel, are staged in LDS as they are,
+// and each tap's 8 channels are gathered from there.
+template <typename T, bool RAW>
 __global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void conv_tile_kernel(ConvParams p) {
   constexpr int PLANES = sizeof(T) == 4 ? 3 : 1;
@@ -63,6 +73,8 @@ void conv_tile_kernel(ConvParams p) {
   const int npix = p.ir * p.ic;
   const int xplane = npix * kXPitch;
   uint16_t* const ws = xs + PLANES * xplane;                       // [2][PLANES][64][32]
+  T* const raw = reinterpret_cast<T*>(ws + 2 * PLANES * WPLANE);   // RAW: [64][rp]
+  const int rp = raw_pitch<T>(p);
 
   // ---- tile coordinates ----
   const int per_img = p.tiles_r * p.tiles_c * p.tiles_co;
@@ -109,9 +121,53 @@ void conv_tile_kernel(ConvParams p) {
     const int row = cw + l32;
     boff[ks] = row * 32 + (((2 * ks + hf) ^ ((row >> 1) & 3)) * 8);
   }
+  const T* const wnb = static_cast<const T*>(p.wn) + (static_cast<int64_t>(mdl) * p.co + co0) * p.ci * taps;
+  const bool wlive = co0 + wco < p.co;
   T wreg[8];
-  auto wload = [&](int64_t koff) {
-    __builtin_memcpy(wreg, __builtin_assume_aligned(wsrc + koff, 16), sizeof(wreg));
+  auto wload = [&](int tap, int t, int c0) {
+    if constexpr (RAW) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int ch = wu * 8 + q;
+        wreg[q] = wlive && c0 + ch < p.ci ? raw[wco * rp + ch * taps + tap] : from_f32<T>(0.f);
+      }
+    } else {
+      const int64_t koff = static_cast<int64_t>(t * taps + tap) * p.ci32 + c0;
+      __builtin_memcpy(wreg, __builtin_assume_aligned(wsrc + koff, 16), sizeof(wreg));
+    }
+  };
+  // RAW: rows of min(32, ci - c0) channels x taps in 16-byte pieces at element alignment (output
+  // channels past the last are not loaded and count as zero)
+  auto stage_raw = [&](int c0) {
+    constexpr int CE = 16 / sizeof(T), U = 8;
+    const int len = (p.ci - c0 < 32 ? p.ci - c0 : 32) * taps, upr = (len + CE - 1) / CE;
+    const int rows = p.co - co0 < 64 ? p.co - co0 : 64;
+    const int units = rows * upr;
+    for (int e0 = tid; e0 < units; e0 += U * kConvThreads) {
+      uint4 v[U];
+      int dst[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int e = e0 + u * kConvThreads;
+        dst[u] = -1;
+        if (e < units) {
+          const int r = e / upr, off = (e - r * upr) * CE;
+          const T* src = wnb + (static_cast<int64_t>(r) * p.ci + c0) * taps + off;
+          if (off + CE <= len) {
+            __builtin_memcpy(&v[u], src, 16);
+          } else {
+            T tail[CE];
+#pragma unroll
+            for (int z = 0; z < CE; ++z) tail[z] = off + z < len ? src[z] : from_f32<T>(0.f);
+            __builtin_memcpy(&v[u], tail, 16);
+          }
+          dst[u] = r * rp + off;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (dst[u] >= 0) *reinterpret_cast<uint4*>(raw + dst[u]) = v[u];
+    }
   };
   auto wstash = [&](int buf) {
     uint4 pl[PLANES];
@@ -140,7 +196,8 @@ void conv_tile_kernel(ConvParams p) {
       const int nks = p.ci - c0 > 16 ? 2 : 1;        // 16-channel steps that hold a channel
       if (staged) __syncthreads();                   // everyone is done with the last chunk
       staged = true;
-      wload(static_cast<int64_t>(t) * taps * p.ci32 + c0);
+      if constexpr (RAW) stage_raw(c0);
+      else wload(0, t, c0);
       // input tile: unit = 8 channels of one pixel, consecutive lanes on consecutive pixels
       {
         const int units = nks * 2 * npix;
@@ -176,12 +233,16 @@ void conv_tile_kernel(ConvParams p) {
           }
         }
       }
+      if constexpr (RAW) {
+        __syncthreads();
+        wload(0, t, c0);
+      }
       wstash(0);
       __syncthreads();
 
       int r = 0, s = 0;                              // tap = r * kw + s
       for (int tap = 0; tap < taps; ++tap) {
-        if (tap + 1 < taps) wload(static_cast<int64_t>(t * taps + tap + 1) * p.ci32 + c0);
+        if (tap + 1 < taps) wload(tap + 1, t, c0);
         const int toff = ((r * p.dh) * p.ic + s * p.dw) * kXPitch;
         const uint16_t* const wt = ws + (tap & 1) * PLANES * WPLANE;
 #pragma unroll
@@ -259,7 +320,9 @@ void conv_tile_kernel(ConvParams p) {
     }
   if (PLANES == 3 && __builtin_amdgcn_ballot_w64(bad) != 0 && co < p.co) {
     // infinities and NaN: the lane's outputs again, in fp32 from memory
-    const T* const wr = wb + static_cast<int64_t>(co) * taps_all * p.ci32;
+    const T* const wr = RAW ? wnb + static_cast<int64_t>(co - co0) * p.ci * taps
+                            : wb + static_cast<int64_t>(co) * taps_all * p.ci32;
+    const int wcs = RAW ? taps : 1;                  // from one input channel to the next
     for (int e = 0; e < 32; ++e) {
       const int px = px0 + (e >> 4) * 32 + ((e & 15) >> 2) * 8 + 4 * hf + (e & 3);
       const int pr = px / p.tc, pc = px - (px / p.tc) * p.tc;
@@ -273,8 +336,8 @@ void conv_tile_kernel(ConvParams p) {
             // a padding pixel is a zero that meets the weight: an infinite weight gives NaN there
             const bool in = hi >= 0 && hi < p.h && wi >= 0 && wi < p.w;
             const T* xp = xb + (static_cast<int64_t>(di) * p.h + (in ? hi : 0)) * p.w + (in ? wi : 0);
-            const T* wp = wr + static_cast<int64_t>((t * p.kh + r) * p.kw + s) * p.ci32;
-            for (int c = 0; c < p.ci; ++c) v += (in ? to_f32(xp[c * p.x_cs]) : 0.f) * to_f32(wp[c]);
+            const T* wp = wr + static_cast<int64_t>((t * p.kh + r) * p.kw + s) * (RAW ? 1 : p.ci32);
+            for (int c = 0; c < p.ci; ++c) v += (in ? to_f32(xp[c * p.x_cs]) : 0.f) * to_f32(wp[c * wcs]);
           }
       cs[(cw + l32) * CPITCH + px] = from_f32<T>(v * alpha + beta);
     }
@@ -317,10 +380,35 @@ bool tile_plan(ConvParams& p, size_t& lds) {
   return best >= 0.0;
 }
 
+// Where the filter bank is read as it is: few tiles (one round of workgroups), at most 9 taps and 160
+// values per output channel.  It saves the packing launch, about 6 us of host time; beyond that staging and
+// gathering the raw rows take longer than packing.  Measured (us for a whole forward, host included,
+// filter bank / packed; models x images, channels, kernel, image):
+//   fp32  30 x 8,   16 ->  64, 1x1, 10 x 10   15.7 / 21.2      bf16  2 x 3, 32 -> 32, 1x3, 389   17.8 / 23.5
+//   bf16  16 x 8,  128 -> 128, 1x1, 8 x 8     14.7 / 20.4      fp32  1 x 3,  1 -> 32, 3x3, 31 x 15  15.5 / 20.9
+//   fp32  16 x 2,   64 ->  64, 3x3, 14 x 14   34.9 / 28.5      fp16  6 x 15, 3 -> 128, 5x5, 8 x 26  22.4 / 21.8
+template <typename T>
+bool raw_fits(const ConvParams& q, size_t* total) {
+  if (q.kd != 1 || q.kh * q.kw > 9 || q.ci * q.kh * q.kw > 160) return false;
+  ConvParams p = q;
+  size_t lds = 0;
+  if (!tile_plan<T>(p, lds)) return false;
+  const size_t in = static_cast<size_t>(p.ir) * p.ic * kXPitch * 2 * (sizeof(T) == 4 ? 3 : 1) +
+                    2 * (sizeof(T) == 4 ? 3 : 1) * 64 * 64;
+  const size_t all = in + static_cast<size_t>(64) * raw_pitch<T>(p) * sizeof(T);
+  *total = all > lds ? all : lds;
+  const int64_t blocks = mul_sat({p.n, p.batch, cdiv(p.ho, p.tr), cdiv(p.wo, p.tc), cdiv(p.co, 64)});
+  int cus = device_cu_count();
+  if (cus <= 0) cus = 256;
+  return *total <= 152 * 1024 && blocks <= cus;
+}
+
 template <typename T>
 int32_t launch_conv_tile(ConvParams p, const char* what, hipStream_t st) {
-  size_t lds = 0;
+  size_t lds = 0, raw_lds = 0;
+  if (!p.wp && !raw_fits<T>(p, &raw_lds)) return 1;
   if (!tile_plan<T>(p, lds)) return 1;
+  if (!p.wp) lds = raw_lds;
   p.fd_plane = make_fastdiv(static_cast<uint32_t>(p.ir * p.ic));
   p.fd_ic = make_fastdiv(static_cast<uint32_t>(p.ic));
   p.tiles_r = static_cast<int>(cdiv(p.ho, p.tr));
@@ -335,7 +423,7 @@ int32_t launch_conv_tile(ConvParams p, const char* what, hipStream_t st) {
   const int64_t nblk = mul_sat({p.n, p.batch, p.dout, p.tiles_r, p.tiles_c, p.tiles_co});
   if (nblk >= 0x7fffffffll) return 1;                // conv_kernel's own limit decides
   p.remap = (nblk % 8 == 0) ? 1 : 0;
-  auto kern = conv_tile_kernel<T>;
+  auto kern = p.wp ? conv_tile_kernel<T, false> : conv_tile_kernel<T, true>;
   if (lds > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
@@ -347,6 +435,12 @@ int32_t launch_conv_tile(ConvParams p, const char* what, hipStream_t st) {
 }
 
 }  // namespace
+
+bool conv_tile_raw(const ConvParams& p, int32_t dtype) {
+  size_t lds = 0;
+  if (dtype == WC_F32) return raw_fits<float>(p, &lds);
+  return raw_fits<bf16>(p, &lds);                    // fp16 likewise: sizes only
+}
 
 int32_t conv_tile(const ConvParams& p, int32_t dtype, const char* what, hipStream_t st) {
   if (dtype == WC_F32) return launch_conv_tile<float>(p, what, st);

@@ -21,7 +21,7 @@ struct ConvParams {
   const void* x;
   int64_t x_sn, x_sb;
   const void* wp;           // packed weights [n][co][kh][kw][ci32]
-  const void* wn;           // or (resident-weight kernel only) the filter bank [n*co][ci][kh][kw]
+  const void* wn;           // or (resident-weight kernel, tile kernel) the filter bank [n*co][ci][kh][kw]
   const void* bias;         // [n*co] or null
   const void* bn_w;         // eval BN params [n*co] (bn_mean null: no BN)
   const void* bn_b;
@@ -118,5 +118,7 @@ __device__ __forceinline__ void conv_store(const ConvParams& p, const T* cs, int
 // The tile kernel (conv_tile.hip); 1 when its tiles do not fit LDS (nothing launched).  p holds the
 // sizes, strides and packed weights; tiles are planned inside.
 int32_t conv_tile(const ConvParams& p, int32_t dtype, const char* what, hipStream_t st);
+// true where the tile kernel reads the filter bank itself (p.wp null)
+bool conv_tile_raw(const ConvParams& p, int32_t dtype);
 
 }  // namespace wc

@@ -668,7 +668,11 @@ def conv2d(*, x: Tensor, weight: Tensor, n: int, c_in: int, c_out: int, kernel, 
             *((0, 0, 0) if residual is None else (residual.data_ptr(), residual.stride(0), residual.stride(1))),
             y.data_ptr(), y.stride(0), y.stride(1), weight.data_ptr())
     a = None
-    if dt == BF16 and not packed:                # only bf16 filters are ever read in their own layout
+    # sizes that one of the two kernels reading the filter bank may take (the tile kernel: short
+    # filters, at least this many workgroups in one round); the library decides
+    if not packed and (c_in * kh * kw <= 160 and kh * kw <= 9 and
+                       n * xs[1] * ((ys[3] * ys[4] + 127) // 128) * ((c_out + 63) // 64) <= 256
+                       or dt == BF16 and kw == 3 and c_in in (32, 64)):
         a = _pack_conv(*head, 0, *tail)
         if not lib().wc_conv2d_direct_weights(ctypes.byref(_ConvArgs.from_buffer_copy(a))):
             a = None

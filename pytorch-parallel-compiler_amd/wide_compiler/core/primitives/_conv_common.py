@@ -3,8 +3,9 @@ Host side of the implicit-GEMM convolution shared by WideConv1d / WideConv2d.
 
 The filters are read from the module's own parameter on every call, as the reference does:
 writes through ``.data`` do not bump a tensor's version counter, so no cache of a derived
-layout keyed on it could see them.  The resident-weight kernel stages the filter bank in its
-natural [N*C_out, C_in, kh, kw] layout; the other kernels take it packed into a K-contiguous
+layout keyed on it could see them.  The resident-weight kernel, and the tile kernel for
+few tiles and short filters, stage the filter bank in its natural [N*C_out, C_in, kh, kw] layout;
+otherwise the kernels take it packed into a K-contiguous
 layout [N, C_out, kh, kw, Ci32] by one small bandwidth kernel per call.  A following eval BatchNorm, residual add and ReLU
 are applied in the conv epilogue when TracedWideModel has fused them (``fused_bn`` /
 ``fused_activation`` / the ``residual`` argument).

@@ -134,3 +134,41 @@ def test_conv_tile_fp32_infinite_weight_meets_padding(hip):
     assert torch.isnan(f[1, :, 7, 0]).all() and torch.isinf(f[1, :, 7, 1:, 1:]).all()
     assert torch.equal(torch.isnan(got), torch.isnan(f))
     assert torch.equal(torch.isinf(got), torch.isinf(f))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,b,ci,co,h,w,kh,kw,stride,pad", [
+    (2, 3, 3, 40, 9, 12, 3, 3, 1, 1),        # rows of 27 values; channels past a tile's first 32
+    (3, 1, 17, 70, 13, 7, 3, 3, 2, 1),       # one channel past an MFMA step, two channel tiles
+    (1, 2, 33, 16, 1, 132, 1, 3, 1, 1),      # one channel in the second chunk
+    (4, 2, 128, 40, 8, 8, 1, 1, 1, 0),       # a tap only, four chunks
+    (2, 1, 53, 24, 21, 7, 3, 1, 2, 1),       # rows of 159 values, a partial chunk
+])
+def test_conv_tile_reads_the_filter_bank(hip, dtype, n, b, ci, co, h, w, kh, kw, stride, pad):
+    """Few tiles: the filters read in their own layout give the packed layout's result bit for bit,
+    also at an address of element alignment; a packed-only size says so."""
+    from wide_compiler import _hip
+    torch.manual_seed(5)
+    x = torch.randn(n, b, ci, h, w, device=DEV).to(dtype)
+    store = (torch.randn(n * co * ci * kh * kw + 1, device=DEV) * 0.1).to(dtype)
+    bias = torch.randn(n * co, device=DEV).to(dtype)
+    ph, pw = (0 if kh == 1 else pad), (0 if kw == 1 else pad)
+    ho, wo = (h + 2 * ph - kh) // stride + 1, (w + 2 * pw - kw) // stride + 1
+    for at in (0, 1):
+        wt = store[at:at + n * co * ci * kh * kw].view(n * co, ci, kh, kw)
+        got = [torch.full((n, b, co, ho, wo), float("nan"), dtype=dtype, device=DEV) for _ in range(2)]
+        packs = []
+        real = _hip.conv_pack_weights
+        try:
+            _hip.conv_pack_weights = lambda *a: (packs.append(1), real(*a))[1]
+            for y, packed in zip(got, (False, True)):
+                _hip.conv2d(x=x, weight=wt, n=n, c_in=ci, c_out=co, kernel=(kh, kw), stride=(stride, stride),
+                            padding=(ph, pw), dilation=(1, 1), y=y, bias=bias, packed=packed)
+        finally:
+            _hip.conv_pack_weights = real
+        assert len(packs) == 1                                # the packed call only
+        assert torch.equal(got[0], got[1])
+        ref = torch.stack([nn.functional.conv2d(x[q].double().cpu(), wt[q * co:(q + 1) * co].double().cpu(),
+                                                bias[q * co:(q + 1) * co].double().cpu(), stride, (ph, pw))
+                           for q in range(n)])
+        _check(got[0].cpu(), ref, ci * kh * kw)
