@@ -6,7 +6,8 @@
 // ahead.  Per tile and wave, with v_mfma_f32_32x32x16:
 //   S^T = K Q^T      lane l holds query l % 32 and the keys 8 (r / 4) + 4 (l / 32) + r % 4 of each
 //                    32-key block in register r
-//   softmax          in the lane: exp2(s * c - max), one FMA and one exponential per score.  The
+//   softmax          in the lane: exp2(s * c - max), one FMA and one exponential per score; the row sum
+//                    takes P in fp32, before it is rounded for P V.  The
 //                    lane halves that share a query exchange their maxima, and O is rescaled,
 //                    only in tiles where a lane of the wave finds a new running maximum.  (Letting
 //                    the base lag behind the maximum by up to 2^8 is 12% faster, but rounds the
@@ -18,7 +19,7 @@
 // Blocks past the diagonal are skipped per wave, and only tiles on the diagonal or past the
 // last key evaluate a mask.
 //
-// Bound by the VALU: about 43 full-rate instructions and 16 exponentials per 32 x 32 scores
+// Bound by the VALU: about 51 full-rate instructions and 16 exponentials per 32 x 32 scores
 // against 256 cycles of MFMA at head dim 64; four waves per SIMD (two from head dim 96 on)
 // overlap the two.  Measured (us, heads x tokens x head dim; before: 16x16x32 MFMAs, V transposed
 // on its way into LDS, a mask and a rescale on every tile):
@@ -55,18 +56,6 @@ __device__ __forceinline__ uint32_t st_pack(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2));
   } else {
     return pack_bf16x2(lo, hi);
-  }
-}
-
-// acc + the two values of a packed pair
-template <typename T>
-__device__ __forceinline__ float st_add2(uint32_t pair, float acc) {
-  if constexpr (std::is_same<T, f16>::value) {
-    const f16x2 ones = {f16(1.0f), f16(1.0f)};
-    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, pair), ones, acc, false);
-  } else {
-    const bf16x2 ones = {bf16(1.0f), bf16(1.0f)};
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), ones, acc, false);
   }
 }
 
@@ -218,17 +207,16 @@ void attn_stream_kernel(AttnParams p) {
     }
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
+      // the row sum takes P before it is rounded for P V, on two independent chains
       uint32_t pk[8];
-#pragma unroll
-      for (int r = 0; r < 8; ++r)
-        pk[r] = st_pack<T>(__builtin_amdgcn_exp2f(__builtin_fmaf(s[b][2 * r], c, -base)),
-                           __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][2 * r + 1], c, -base)));
-      // the row sum takes the rounded P that P V uses, on two independent chains
       float l0 = 0.f, l1 = 0.f;
 #pragma unroll
-      for (int r = 0; r < 8; r += 2) {
-        l0 = st_add2<T>(pk[r], l0);
-        l1 = st_add2<T>(pk[r + 1], l1);
+      for (int r = 0; r < 8; ++r) {
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][2 * r], c, -base));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][2 * r + 1], c, -base));
+        l0 += p0;
+        l1 += p1;
+        pk[r] = st_pack<T>(p0, p1);
       }
       lrun += l0 + l1;
 #pragma unroll

@@ -108,3 +108,27 @@ def test_stream_non_finite_values(hip):
     assert nan[1, :, dh:].all() and not nan[1, :, :dh].any()
     assert torch.isinf(got[2, :, 1]).all() and torch.equal(got[2, :, 2:], clean[2, :, 2:])
     assert torch.equal(got[3], clean[3])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dh,skv,causal", [(64, 2047, False), (64, 2048, True), (40, 1000, False), (128, 513, False)])
+def test_stream_row_sum_is_32_bit(hip, dh, skv, causal, dtype):
+    """The row sum takes P before it is rounded for P V.  One key holds the row's largest score and the
+    only non-zero value, so P V is exactly 1 and the output 1 / l; the other keys of a row all have
+    the same P, whose rounding, were it in l, would not average out.  Bar: half an ulp of the output
+    type, and 2^-18 for fp32's share (the exponential, its argument, 2,048 additions in two chains)."""
+    torch.manual_seed(dh + skv)
+    nb, sq = 2, 256 if not causal else skv
+    q = torch.zeros(nb, sq, dh, device=DEV)
+    q[:, :, 0] = torch.rand(nb, sq, device=DEV) * 4.0 + 0.5
+    k = torch.zeros(nb, skv, dh, device=DEV)
+    k[:, 0, 0] = dh ** 0.5
+    v = torch.zeros(nb, skv, dh, device=DEV)
+    v[:, 0] = 1.0
+    q, k, v = (t.to(dtype) for t in (q, k, v))
+    got = _attend(q, k, v, 1, causal, False).double()
+    d = q[:, :, 0].double() * k[0, 0, 0].double() * dh ** -0.5
+    others = torch.arange(sq, device=DEV).double() if causal else float(skv - 1)
+    ref = (1.0 / (1.0 + others * torch.exp(-d)))[:, :, None]
+    half_ulp = torch.exp2(torch.floor(torch.log2(ref))) * (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11)
+    assert ((got - ref).abs() <= half_ulp + 2.0 ** -18 * ref).all()
