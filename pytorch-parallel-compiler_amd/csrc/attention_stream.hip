@@ -138,9 +138,10 @@ void attn_stream_kernel(AttnParams p) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) oacc[d][e] = 0.f;
   const float c = p.scale_log2;
-  // base: subtracted from the scaled scores (0 until the first block sets it); lrun: this lane
-  // half's part of the row sum
+  // base: subtracted from the scaled scores, 0 until the query has met a score above -infinity (fresh;
+  // its sums are zero until then); lrun: this lane half's part of the row sum
   float base = 0.f, lrun = 0.f;
+  bool fresh = true;
 
   int kend = p.skv;
   if (CAUSAL) {
@@ -193,17 +194,18 @@ void attn_stream_kernel(AttnParams p) {
                               __builtin_fmaxf(__builtin_fmaxf(m3, m4), s[b][15]));
     }
     float bm = (NB == 2 ? __builtin_fmaxf(mx[0], mx[NB - 1]) : mx[0]) * c;
-    const bool first = k0 == 0;
-    if (__builtin_amdgcn_ballot_w64(first || bm > base) != 0) {
+    if (__builtin_amdgcn_ballot_w64(fresh || bm > base) != 0) {
       bm = __builtin_fmaxf(bm, __shfl_xor(bm, 32, 64));
-      const float nbase = (first || bm > base) && bm > -INFINITY ? bm : base;
-      if (!first) {
-        const float alpha = __builtin_amdgcn_exp2f(base - nbase);
+      const bool up = (fresh || bm > base) && bm > -INFINITY;
+      const float nbase = up ? bm : base;
+      if (k0 != 0) {
+        const float alpha = fresh ? 1.0f : __builtin_amdgcn_exp2f(base - nbase);
 #pragma unroll
         for (int d = 0; d < DT; ++d) oacc[d] *= alpha;
         lrun *= alpha;
       }
       base = nbase;
+      fresh = fresh && !up;
     }
 #pragma unroll
     for (int b = 0; b < NB; ++b) {

@@ -132,3 +132,33 @@ def test_stream_row_sum_is_32_bit(hip, dh, skv, causal, dtype):
     ref = (1.0 / (1.0 + others * torch.exp(-d)))[:, :, None]
     half_ulp = torch.exp2(torch.floor(torch.log2(ref))) * (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11)
     assert ((got - ref).abs() <= half_ulp + 2.0 ** -18 * ref).all()
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("dtype,blocked", [(torch.bfloat16, 64), (torch.bfloat16, 150), (torch.float16, 128)])
+def test_stream_first_scores_are_minus_infinity(hip, dtype, blocked, causal):
+    """Keys whose score is -infinity (an overflow in bf16, an infinite key in fp16) weigh nothing, also when they
+    come first and the scores after them lie far below zero: the row's maximum is the largest of the
+    finite ones.  Every score is the same but theirs, so the output is the mean of the other values."""
+    heads, dh, s = 2, 64, 260
+    torch.manual_seed(blocked)
+    q = torch.zeros(2, s, heads, dh, device=DEV)
+    k = torch.zeros(2, s, heads, dh, device=DEV)
+    if dtype == torch.bfloat16:
+        q[..., 0] = 1e20
+        k[..., 0] = -2e-17                                  # scores of -250
+        k[:, :blocked, :, 0] = -1e20
+    else:
+        q[..., 0] = 100.0
+        k[..., 0] = -20.0
+        k[:, :blocked, :, 0] = -float("inf")
+    q, k = (t.view(2, s, heads * dh).to(dtype) for t in (q, k))
+    v = torch.randn(2, s, heads * dh, device=DEV).to(dtype)
+    got = _attend(q, k, v, heads, causal, False).double()
+    sums = v.double()[:, blocked:].cumsum(1)
+    if causal:
+        ref = sums / torch.arange(1, s - blocked + 1, device=DEV).double()[:, None]
+        got = got[:, blocked:]                              # rows that see no other key have no defined value
+    else:
+        ref = (sums[:, -1:] / (s - blocked)).expand(2, s, heads * dh)
+    assert _err(got, ref) <= BAR[dtype]
