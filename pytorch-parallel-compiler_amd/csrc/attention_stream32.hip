@@ -8,8 +8,9 @@
 // split on their way into LDS, and V^T comes from the row-major planes through
 // ds_read_b64_tr_b16.  Softmax, maxima and row sums are fp32 as before.
 //
-// Infinities: when a value of Q, K or V cannot be carried by the planes, the workgroup computes
-// its queries again with fp32 multiply-adds from memory.
+// What the planes do not carry: a workgroup that met a Q or K of 2^56 or more, where a score could overflow
+// or the planes' absolute error could count, or a V of 2^100 or more, where a sum could, computes its
+// queries again on the fp32 MFMA, straight from memory.
 //
 // Bound by the VALU (softmax, splitting P: about 2,000 cycles per wave and tile against 1,536 of
 // MFMAs at head dim 32) and, for short sequences, by the latency of the first loads.  Measured (us,
@@ -19,7 +20,9 @@
 //     64 x 2048 x 64          657 -> 374   [8.7e-7 -> 3.5e-7]  (184 TFLOP/s)
 //     64 x 2048 x 64 causal   540 -> 214   [4.0e-7 -> 1.7e-7]
 //    512 x 512 x 32           180 -> 107
-// Head dims past 64 would spill (Q and O planes of 128 columns) and keep the general kernel.
+// The fp32 way takes about 5 times as long (64 x 2048 x 64: 372 and then 1,790; the general kernel 657).
+// Registers: no scratch at head dims up to 32, 7 (causal 10) spilled at 64; head dims past 64 (Q and O planes of
+// 128 columns) would spill far more and keep the general kernel.
 #include "wc_attn.h"
 
 namespace wc {
@@ -30,6 +33,7 @@ typedef short i16x8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 
 constexpr int kS32Threads = 256;       // four waves of 32 queries
+constexpr float kBigV = 0x1p100f;      // below it no sum of 2^27 values overflows
 
 template <int DHP, bool CAUSAL>
 __global__ __launch_bounds__(kS32Threads) __attribute__((amdgpu_waves_per_eu(DHP == 32 ? 3 : 2)))
@@ -43,7 +47,7 @@ void attn_stream32_kernel(AttnParams p) {
   constexpr int NBUF = DHP == 32 ? 2 : 1;            // what leaves three workgroups per CU their LDS
   static_assert(2 * UN % NT == 0 && UN % NT == 0, "units divide evenly");
   __shared__ __attribute__((aligned(16))) uint16_t lds[NBUF][2][3][TILE];   // K planes, V planes
-  __shared__ int bad_flag;
+  __shared__ int odd_flag;
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int l32 = lane & 31, hf = lane >> 5;
@@ -57,10 +61,10 @@ void attn_stream32_kernel(AttnParams p) {
   float* ob = static_cast<float*>(p.o) + nb * p.o_sb + static_cast<int64_t>(h) * dh;
   const int q0 = qt * 128 + wave * 32;               // the wave's first query
   const int q = q0 + l32;                            // the lane's query
-  if (tid == 0) bad_flag = 0;
+  if (tid == 0) odd_flag = 0;
   __syncthreads();
 
-  bool bad = false;
+  bool odd = false;                                  // met what the planes do not carry
   // 8 values from src, those at column c and past it that exist
   auto load8 = [&](const float* src, int c, float (&v)[8]) {
     f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
@@ -72,11 +76,6 @@ void attn_stream32_kernel(AttnParams p) {
       v[4 + e] = b[e];
     }
   };
-  auto note = [&](const float (&v)[8]) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) bad |= __builtin_fabsf(v[e]) > kPlaneMax;
-  };
-
   // ---- Q^T planes (B operand of S^T): query l32, dims 16 k + 8 hf .. + 8 ----
   bf16x8 qf[NKS][3];
   {
@@ -85,7 +84,7 @@ void attn_stream32_kernel(AttnParams p) {
     for (int k = 0; k < NKS; ++k) {
       float v[8];
       load8(qr, 16 * k + 8 * hf, v);
-      note(v);
+      odd |= abs_max8(v) >= kPlaneSafe;
       uint4 pl[3];
       split_planes(v, pl);
 #pragma unroll
@@ -113,7 +112,7 @@ void attn_stream32_kernel(AttnParams p) {
       const bool isv = u >= PT / 2;
       const int e = tid + (isv ? u - PT / 2 : u) * NT;
       const int key = e / UPR, c = e % UPR;
-      note(reg[u]);
+      odd |= abs_max8(reg[u]) >= (isv ? kBigV : kPlaneSafe);
       uint4 pl[3];
       split_planes(reg[u], pl);
       const int at = isv ? v_at<DHP>(key, c * 8) : k_at<DHP>(key, c);
@@ -260,51 +259,90 @@ void attn_stream32_kernel(AttnParams p) {
     }
   }
 
-  // ---- O = (O^T / l)^T: lane holds query l32, dims 32 d + 8 (r / 4) + 4 hf + r % 4 ----
+  // the lane's coordinates anew: the key loop then keeps no registers for them
+  int ln = 0;
+  asm volatile("" : "+v"(ln));
+  ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, ln));
+  const int el = ln & 31, eh = ln >> 5, eq0 = __builtin_amdgcn_readfirstlane(q0), eq = eq0 + el;
+
+  // ---- again in fp32: each wave its 32 queries, 32 keys at a time, operands from memory.  k-steps pair
+  // dims d and d + 4 (dh % 4 == 0), keys key and key + 4. ----
+  if (odd) odd_flag = 1;
+  __syncthreads();
+  if (odd_flag != 0 && eq0 < p.sq) {
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) oacc[d][e] = 0.f;
+    base = lrun = 0.f;
+    bool fresh = true;                               // no score above -infinity yet
+    const float* const qr = qb + static_cast<int64_t>(eq < p.sq ? eq : p.sq - 1) * p.q_ss;
+    const int kw = CAUSAL && eq0 + 32 < kend ? eq0 + 32 : kend;
+    for (int k0 = 0; k0 < kw; k0 += 32) {
+      f32x16 s;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s[e] = 0.f;
+      const int krow = k0 + el < p.skv ? k0 + el : p.skv - 1;       // past the last: masked below
+      const float* const kr = kb + static_cast<int64_t>(krow) * p.k_ss;
+      for (int d0 = 0; d0 < dh; d0 += 8) {
+        f32x4 kv = {0.f, 0.f, 0.f, 0.f}, qv = kv;
+        if (d0 + 4 * eh < dh) {
+          kv = *reinterpret_cast<const f32x4*>(kr + d0 + 4 * eh);
+          qv = *reinterpret_cast<const f32x4*>(qr + d0 + 4 * eh);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[e], qv[e], s, 0, 0, 0);
+      }
+      float bm = -INFINITY;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = k0 + (r >> 2) * 8 + 4 * eh + (r & 3);
+        if (key >= p.skv || (CAUSAL && key > eq)) s[r] = -INFINITY;
+        bm = __builtin_fmaxf(bm, s[r]);
+      }
+      bm *= c;
+      bm = __builtin_fmaxf(bm, __shfl_xor(bm, 32, 64));
+      const bool up = (fresh || bm > base) && bm > -INFINITY;
+      const float nbase = up ? bm : base;
+      const float alpha = fresh ? 1.0f : __builtin_amdgcn_exp2f(base - nbase);
+#pragma unroll
+      for (int d = 0; d < DT; ++d) oacc[d] *= alpha;
+      base = nbase;
+      fresh = fresh && !up;
+      float l0 = 0.f, l1 = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float pr = __builtin_amdgcn_exp2f(s[r] * c - base);
+        if (r & 1) l1 += pr;
+        else l0 += pr;
+        const int key = k0 + (r >> 2) * 8 + 4 * eh + (r & 3);
+        const float* const vr = vb + static_cast<int64_t>(key < p.skv ? key : p.skv - 1) * p.v_ss;
+#pragma unroll
+        for (int d = 0; d < DT; ++d) {
+          const float v = key < p.skv && 32 * d + el < dh ? vr[32 * d + el] : 0.f;
+          oacc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(v, pr, oacc[d], 0, 0, 0);
+        }
+      }
+      lrun = lrun * alpha + (l0 + l1);
+    }
+  }
+
+  // ---- O = (O^T / l)^T: lane holds query el, dims 32 d + 8 (r / 4) + 4 eh + r % 4 ----
   const float lt = lrun + __shfl_xor(lrun, 32, 64);
-  float* const orow = ob + static_cast<int64_t>(q < p.sq ? q : 0) * p.o_ss;
-  if (q < p.sq) {
+  if (eq < p.sq) {
+    float* const orow = ob + static_cast<int64_t>(eq) * p.o_ss;
     const float inv = lt > 0.f ? 1.0f / lt : (lt == 0.f ? 0.f : lt);      // NaN stays NaN
 #pragma unroll
     for (int d = 0; d < DT; ++d)
 #pragma unroll
       for (int g4 = 0; g4 < 4; ++g4) {
-        const int col = 32 * d + 8 * g4 + 4 * hf;
+        const int col = 32 * d + 8 * g4 + 4 * eh;
         if (col < dh) {                              // dh % 4 == 0: whole groups of 4
           const f32x4 v = {oacc[d][4 * g4] * inv, oacc[d][4 * g4 + 1] * inv, oacc[d][4 * g4 + 2] * inv,
                            oacc[d][4 * g4 + 3] * inv};
           __builtin_memcpy(orow + col, &v, 16);      // output rows at element alignment
         }
       }
-  }
-
-  // ---- a value the planes do not carry: the workgroup's queries again, in fp32 from memory; the
-  // two lanes of a query take half of the groups of 4 dims each ----
-  if (bad) bad_flag = 1;
-  __syncthreads();
-  if (bad_flag != 0 && q < p.sq) {
-    const float* qr = qb + static_cast<int64_t>(q) * p.q_ss;
-    const int keys = CAUSAL ? (q + 1 < p.skv ? q + 1 : p.skv) : p.skv;
-    auto score = [&](int key) {
-      const float* kr = kb + static_cast<int64_t>(key) * p.k_ss;
-      float t = 0.f;
-      for (int d = 0; d < dh; ++d) t += qr[d] * kr[d];
-      return t * c;
-    };
-    float m = -INFINITY;
-    for (int key = 0; key < keys; ++key) m = __builtin_fmaxf(m, score(key));
-    if (m == -INFINITY) m = 0.f;
-    for (int col = 4 * hf; col < dh; col += 8) {
-      float l = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
-      for (int key = 0; key < keys; ++key) {
-        const float pr = __builtin_amdgcn_exp2f(score(key) - m);
-        const float* vr = vb + static_cast<int64_t>(key) * p.v_ss + col;
-        l += pr;
-        for (int e = 0; e < 4; ++e) o[e] += pr * vr[e];
-      }
-      const float inv = l > 0.f ? 1.0f / l : (l == 0.f ? 0.f : l);
-      for (int e = 0; e < 4; ++e) orow[col + e] = o[e] * inv;
-    }
   }
 }
 
@@ -321,7 +359,8 @@ int32_t launch_s32(AttnParams p, hipStream_t st) {
 }  // namespace
 
 int32_t attn_stream32(const AttnParams& p, hipStream_t st) {
-  if (p.dh % 4 != 0 || p.dh > 64 || p.mask || !(p.scale_log2 > 0.f && p.scale_log2 < INFINITY)) return 1;
+  // a scale of 2^30 could lift what the planes lose of a score (kPlaneSafe) to what counts
+  if (p.dh % 4 != 0 || p.dh > 64 || p.mask || !(p.scale_log2 > 0.f && p.scale_log2 < 0x1p30f)) return 1;
   return p.dh <= 32 ? launch_s32<32>(p, st) : launch_s32<64>(p, st);
 }
 

@@ -112,6 +112,21 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 // v2 = v - v0 - v1: every bit of a normal fp32 value above 2^-109.  Infinities, NaN and values
 // above kPlaneMax (they may round to infinity) leave NaN in the planes.
 constexpr float kPlaneMax = 3.38e38f;
+// Below kPlaneSafe the planes of a dot product's operands need no further look where only the sum's
+// absolute error counts (a score, a gate): products and their sums of up to 2^14 terms stay under
+// 2^127, so none overflows, and what the planes of a value under 2^-109 lose, at most 2^-134 of each,
+// stays under 2^-64.
+constexpr float kPlaneSafe = 0x1p56f;
+
+// the largest magnitude of 8 values (v_max3_f32; a NaN among them is ignored or makes it NaN)
+__device__ __forceinline__ float abs_max8(const float (&v)[8]) {
+  float m;
+  asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(m) : "v"(v[0]), "v"(v[1]), "v"(v[2]));
+  asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(m) : "v"(m), "v"(v[3]), "v"(v[4]));
+  asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(m) : "v"(m), "v"(v[5]), "v"(v[6]));
+  asm("v_max_f32_e64 %0, %1, |%2|" : "=v"(m) : "v"(m), "v"(v[7]));
+  return m;
+}
 __device__ __forceinline__ void split_planes(const float (&v)[8], uint4 (&pl)[3]) {
   float f[8];
 #pragma unroll

@@ -81,3 +81,46 @@ def test_stream32_non_finite_values(hip, causal):
         assert (got[b][:, rest] - clean[b][:, rest]).abs().max().item() <= 1e-5
     assert torch.equal(torch.isnan(got[4, 9]), torch.isnan(general[4, 9]))
     assert torch.equal(got[5], clean[5])
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("qv,kv", [(1.003e3, -3e38), (3.01e20, -3.01e20), (-2.0 ** 90, 2.0 ** 60)])
+def test_stream32_scores_that_overflow(hip, qv, kv, causal):
+    """Finite operands whose product overflows to -infinity: the key weighs nothing, as in fp32
+    arithmetic, and the row's other keys share the weight."""
+    torch.manual_seed(11)
+    heads, dh, s = 2, 64, 200
+    q = torch.full((2, s, heads * dh), qv, device=DEV)
+    k = torch.randn(2, s, heads * dh, device=DEV) / abs(qv)
+    v = torch.randn(2, s, heads * dh, device=DEV)
+    k[:, 5::7] = kv
+    ref = _ref(q, k, v, heads, causal)
+    got, general = _attend(q, k, v, heads, causal, False), _attend(q, k, v, heads, causal, True)
+    assert not torch.isnan(general).any() and not torch.isnan(got).any()
+    assert _err(got, ref) <= _err(general, ref) + 2.0 ** -24
+
+
+def test_stream32_values_that_overflow(hip):
+    """Values whose unnormalised sum exceeds fp32: infinite, as in the general kernel.  (1.4965 x 2^127 rounds up
+    as a bf16, and enough keys take the sum of those roundings to the other infinity.)"""
+    heads, dh, s = 1, 32, 4000
+    q, k = (torch.zeros(1, s, heads * dh, device=DEV) for _ in range(2))
+    v = torch.full((1, s, heads * dh), 1.4965 * 2.0 ** 127, device=DEV)
+    v[:, :, 1] *= -1.0
+    v[:, :, 2] = 1.0
+    got, general = _attend(q, k, v, heads, False, False), _attend(q, k, v, heads, False, True)
+    assert torch.isinf(general[:, :, :2]).all()
+    assert torch.equal(got[:, :, :2], general[:, :, :2])
+    assert ((got[:, :, 2] - 1.0).abs() <= 2.0 ** -20).all()
+
+
+@pytest.mark.parametrize("qs", [2.0 ** -115, 2.0 ** -122, 2.0 ** 100])
+def test_stream32_queries_and_keys_far_apart(hip, qs):
+    """Queries and keys of opposite scales, ordinary scores."""
+    torch.manual_seed(13)
+    heads, dh, s = 2, 64, 140
+    q, k, v = (torch.randn(2, s, heads * dh, device=DEV) for _ in range(3))
+    q, k = q * qs, k / qs
+    ref = _ref(q, k, v, heads, False)
+    e, general = _err(_attend(q, k, v, heads, False, False), ref), _err(_attend(q, k, v, heads, False, True), ref)
+    assert e <= general + 2.0 ** -24, (e, general)
