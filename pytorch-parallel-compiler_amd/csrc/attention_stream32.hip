@@ -9,8 +9,8 @@
 // ds_read_b64_tr_b16.  Softmax, maxima and row sums are fp32 as before.
 //
 // What the planes do not carry: a workgroup that met a Q or K of 2^56 or more, where a score could overflow
-// or the planes' absolute error could count, or a V of 2^100 or more, where a sum could, computes its
-// queries again on the fp32 MFMA, straight from memory.
+// or the planes' absolute error could count, or a V of 2^100 or more, where a sum could, or a non-zero V under
+// 2^-110, computes its queries again on the fp32 MFMA, straight from memory.
 //
 // Bound by the VALU (softmax, splitting P: about 2,000 cycles per wave and tile against 1,536 of
 // MFMAs at head dim 32) and, for short sequences, by the latency of the first loads.  Measured (us,
@@ -112,7 +112,7 @@ void attn_stream32_kernel(AttnParams p) {
       const bool isv = u >= PT / 2;
       const int e = tid + (isv ? u - PT / 2 : u) * NT;
       const int key = e / UPR, c = e % UPR;
-      odd |= abs_max8(reg[u]) >= (isv ? kBigV : kPlaneSafe);
+      odd |= abs_max8(reg[u]) >= (isv ? kBigV : kPlaneSafe) || (isv && below_planes(reg[u]));
       uint4 pl[3];
       split_planes(reg[u], pl);
       const int at = isv ? v_at<DHP>(key, c * 8) : k_at<DHP>(key, c);

@@ -108,25 +108,41 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
 
-// 8 floats as three bf16 planes, v = v0 + v1 + v2 with v0 = bf16(v), v1 = bf16(v - v0),
-// v2 = v - v0 - v1: every bit of a normal fp32 value above 2^-109.  Infinities, NaN and values
-// above kPlaneMax (they may round to infinity) leave NaN in the planes.
-constexpr float kPlaneMax = 3.38e38f;
+// The range of values that split_planes (below) carries.
+constexpr float kPlaneMax = 3.38e38f, kPlaneMin = 0x1p-110f;
 // Below kPlaneSafe the planes of a dot product's operands need no further look where only the sum's
 // absolute error counts (a score, a gate): products and their sums of up to 2^14 terms stay under
-// 2^127, so none overflows, and what the planes of a value under 2^-109 lose, at most 2^-134 of each,
-// stays under 2^-64.
+// 2^127, so none overflows, and what the planes of values under kPlaneMin lose stays under 2^-63.
 constexpr float kPlaneSafe = 0x1p56f;
 
-// the largest magnitude of 8 values (v_max3_f32; a NaN among them is ignored or makes it NaN)
-__device__ __forceinline__ float abs_max8(const float (&v)[8]) {
-  float m;
-  asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(m) : "v"(v[0]), "v"(v[1]), "v"(v[2]));
-  asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(m) : "v"(m), "v"(v[3]), "v"(v[4]));
-  asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(m) : "v"(m), "v"(v[5]), "v"(v[6]));
-  asm("v_max_f32_e64 %0, %1, |%2|" : "=v"(m) : "v"(m), "v"(v[7]));
+// the largest of m and the magnitudes of 8 values (v_max3_f32; NaN among them are ignored, or take the
+// place of the two before them)
+__device__ __forceinline__ float abs_max8(const float (&v)[8], float m = 0.f) {
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(m) : "v"(m), "v"(v[e]), "v"(v[e + 1]));
   return m;
 }
+
+// true when one of 8 values is non-zero and under kPlaneMin: four v_min3_f32, and a closer look only where
+// a lane of the wave holds such a value or a zero
+__device__ __forceinline__ bool below_planes(const float (&v)[8]) {
+  float m;
+  asm("v_min3_f32 %0, |%1|, |%2|, |%3|" : "=v"(m) : "v"(v[0]), "v"(v[1]), "v"(v[2]));
+  asm("v_min3_f32 %0, %1, |%2|, |%3|" : "=v"(m) : "v"(m), "v"(v[3]), "v"(v[4]));
+  asm("v_min3_f32 %0, %1, |%2|, |%3|" : "=v"(m) : "v"(m), "v"(v[5]), "v"(v[6]));
+  asm("v_min_f32_e64 %0, %1, |%2|" : "=v"(m) : "v"(m), "v"(v[7]));
+  bool below = false;
+  if (__builtin_amdgcn_ballot_w64(m < kPlaneMin) != 0) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) below |= __builtin_fabsf(v[e]) < kPlaneMin && v[e] != 0.f;
+  }
+  return below;
+}
+
+// 8 floats as three bf16 planes, v = v0 + v1 + v2 with v0 = bf16(v), v1 = bf16(v - v0),
+// v2 = v - v0 - v1: every bit of an fp32 value from kPlaneMin on.  Below it bits fall under 2^-133, the
+// smallest bf16, and up to 2^-134 is lost.  Infinities, NaN and values above kPlaneMax (they may
+// round to infinity) leave NaN in the planes.
 __device__ __forceinline__ void split_planes(const float (&v)[8], uint4 (&pl)[3]) {
   float f[8];
 #pragma unroll

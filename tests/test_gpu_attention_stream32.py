@@ -114,6 +114,24 @@ def test_stream32_values_that_overflow(hip):
     assert ((got[:, :, 2] - 1.0).abs() <= 2.0 ** -20).all()
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("vs", [2.0 ** -112, 2.0 ** -120, 2.0 ** -126, 2.0 ** -138])
+def test_stream32_small_values(hip, vs, causal):
+    """Values below what three bf16 planes carry, in some columns of one head: those columns' outputs keep the
+    general kernel's error, and 2^-148 for the steps of subnormal numbers."""
+    torch.manual_seed(12)
+    heads, dh, s = 2, 40, 150
+    q, k, v = (torch.randn(2, s, heads * dh, device=DEV) for _ in range(3))
+    v[0, :, 3:9] *= vs
+    v[1, :, dh:] *= vs
+    ref = _ref(q, k, v, heads, causal)
+    got, general = (_attend(q, k, v, heads, causal, m).double() for m in (False, True))
+    for cols in ((0, slice(3, 9)), (1, slice(dh, 2 * dh)), (0, slice(9, 2 * dh))):
+        g, e, r = (t[cols[0], :, cols[1]] for t in (got, general, ref))
+        slack = 2.0 ** -24 + 2.0 ** -148 * r.numel() ** 0.5 / r.norm().item()
+        assert _err(g, r) <= _err(e, r) + slack, cols
+
+
 @pytest.mark.parametrize("qs", [2.0 ** -115, 2.0 ** -122, 2.0 ** 100])
 def test_stream32_queries_and_keys_far_apart(hip, qs):
     """Queries and keys of opposite scales, ordinary scores."""
