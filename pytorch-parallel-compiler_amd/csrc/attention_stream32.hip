@@ -112,7 +112,8 @@ void attn_stream32_kernel(AttnParams p) {
       const bool isv = u >= PT / 2;
       const int e = tid + (isv ? u - PT / 2 : u) * NT;
       const int key = e / UPR, c = e % UPR;
-      odd |= abs_max8(reg[u]) >= (isv ? kBigV : kPlaneSafe) || (isv && below_planes(reg[u]));
+      odd |= abs_max8(reg[u]) >= (isv ? kBigV : kPlaneSafe);
+      if (isv && __builtin_amdgcn_ballot_w64(abs_min8(reg[u]) < kPlaneMin) != 0) odd |= below_planes(reg[u]);
       uint4 pl[3];
       split_planes(reg[u], pl);
       const int at = isv ? v_at<DHP>(key, c * 8) : k_at<DHP>(key, c);

@@ -16,8 +16,11 @@
 // for 16 values of k: measured against fp64 the result is closer than the fp32 MFMA's.
 // Infinities and NaN (and values that round up to infinity in bf16) leave a NaN or an infinity
 // in the accumulator; a wave that finds one recomputes its tile with the fp32 MFMA from memory,
-// so such inputs give exactly what fp32 arithmetic gives.  (Below 2^-109 the third plane leaves
-// bf16's exponent range: an absolute error under 2^-133 of such a value.)
+// so such inputs give exactly what fp32 arithmetic gives.  Operands under 2^-110 the planes hold in
+// fewer bits.  That can show in a result under kPlaneSmall, or beside an operand of kPlaneBig or more: a
+// workgroup with either looks for such operands (its staged rows once more, a fifth of a tile's time) and
+// if it finds one recomputes too.  Tracking the largest operand costs 1-2 %; testing each for being
+// small instead cost 2-4, and 4-7 where zeros are common.
 //
 // What bounds it: the MFMAs at the clock that random operands allow (a large bf16 product reaches
 // 1.25 PFLOP/s on this chip, a sixth of which is 208 TFLOP/s in fp32), and for short k the first
@@ -72,14 +75,17 @@ struct TileCfg {
   static constexpr int LDS = STAGE_BYTES > EPI_BYTES ? STAGE_BYTES : EPI_BYTES;
 };
 
-// At least two waves per SIMD (registers), so that two workgroups share a CU.
+// At least two waves per SIMD (registers), so that two workgroups share a CU; three and, for the 64 x 64
+// tile, five in fp32, which the compiler misses by a few registers if left alone.
 template <typename TA, typename TC, typename TB, int FM, int FN>
-__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ __launch_bounds__(kTileThreads)
+__attribute__((amdgpu_waves_per_eu(sizeof(TA) != 4 ? 2 : FM * FN == 1 ? 5 : 3)))
 void gemm_tile_kernel(GemmParams p) {
   using C = TileCfg<TA, FM, FN>;
   constexpr int PLANES = C::PLANES, BK = C::BK, UPR = C::UPR, BM = C::BM, BN = C::BN, UPT = C::UPT;
   __shared__ __attribute__((aligned(16))) char smem[C::LDS];
   uint16_t* const lds = reinterpret_cast<uint16_t*>(smem);
+  __shared__ int flags[2];                           // fp32: look at the operands again; compute again
 
   // tile coordinates (XCD-aware: consecutive tiles, which share operands, run on one XCD)
   const int tiles_per_model = p.tiles_m * p.tiles_o;
@@ -141,6 +147,7 @@ void gemm_tile_kernel(GemmParams p) {
       }
     }
   };
+  float top = 0.f;                                   // fp32: the largest operand this thread has staged
   auto stash = [&]() {
 #pragma unroll
     for (int q = 0; q < UPT; ++q) {
@@ -150,6 +157,7 @@ void gemm_tile_kernel(GemmParams p) {
       } else {
         float f[8];
         __builtin_memcpy(f, &reg[q], sizeof(f));
+        top = abs_max8(f, top);
         uint4 pl[3];
         split_planes(f, pl);
 #pragma unroll
@@ -176,6 +184,7 @@ void gemm_tile_kernel(GemmParams p) {
 #pragma unroll
   for (int e = 0; e < 16; ++e) low[e] = 0.f;
 
+  if (PLANES == 3 && tid < 2) flags[tid] = 0;
   const int ksteps = (p.k + BK - 1) / BK;
   if (ksteps > 0) {
     fetch(0);
@@ -219,7 +228,7 @@ void gemm_tile_kernel(GemmParams p) {
 
   if constexpr (PLANES == 3) {
     if constexpr (LOW) acc[0][0] += low;
-    // infinities and NaN: the wave's tile again, with the fp32 MFMA straight from memory
+    // what the planes do not carry: the wave's tile again, with the fp32 MFMA straight from memory
     bool bad = false;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
@@ -227,6 +236,30 @@ void gemm_tile_kernel(GemmParams p) {
       for (int j = 0; j < FN; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) bad |= !(__builtin_fabsf(acc[i][j][e]) <= 3.402823466e38f);
+    bool ask = top >= kPlaneBig;                     // could an operand under kPlaneMin show?
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) ask |= __builtin_fabsf(acc[i][j][e]) < kPlaneSmall;
+    if (ask) flags[0] = 1;
+    __syncthreads();
+    if (flags[0] != 0) {
+      bool below = false;
+      for (int kt = 0; kt < ksteps; ++kt) {
+        fetch(kt * BK);
+#pragma unroll
+        for (int q = 0; q < UPT; ++q) {
+          float f[8];
+          __builtin_memcpy(f, &reg[q], sizeof(f));
+          below |= below_planes(f);
+        }
+      }
+      if (below) flags[1] = 1;
+      __syncthreads();
+      bad |= flags[1] != 0;
+    }
     if (__builtin_amdgcn_ballot_w64(bad) != 0) {
       const TA* ar[FM];
       const TA* wr[FN];
@@ -240,18 +273,31 @@ void gemm_tile_kernel(GemmParams p) {
         for (int j = 0; j < FN; ++j)
 #pragma unroll
           for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-      for (int k0 = 0; k0 < p.k; k0 += 2) {
-        const int k = k0 + hf;
-        float av[FM], wv[FN];
+      // 8 values of k at a time, 4 of each lane half: a step pairs k and k + 4
+      auto load4 = [&](const TA* row, int k) {
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+        if (k + 4 <= p.k) {
+          __builtin_memcpy(&v, row + k, 16);         // element alignment
+        } else {
 #pragma unroll
-        for (int i = 0; i < FM; ++i) av[i] = k < p.k ? to_f32(ar[i][k]) : 0.f;
+          for (int e = 0; e < 4; ++e)
+            if (k + e < p.k) v[e] = to_f32(row[k + e]);
+        }
+        return v;
+      };
+      for (int k0 = 0; k0 < p.k; k0 += 8) {
+        f32x4 av[FM], wv[FN];
 #pragma unroll
-        for (int j = 0; j < FN; ++j) wv[j] = k < p.k ? to_f32(wr[j][k]) : 0.f;
+        for (int i = 0; i < FM; ++i) av[i] = load4(ar[i], k0 + 4 * hf);
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
+        for (int j = 0; j < FN; ++j) wv[j] = load4(wr[j], k0 + 4 * hf);
 #pragma unroll
-          for (int j = 0; j < FN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[j], av[i], acc[i][j], 0, 0, 0);
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[j][e], av[i][e], acc[i][j], 0, 0, 0);
       }
     }
   }

@@ -115,6 +115,11 @@ constexpr float kPlaneMax = 3.38e38f, kPlaneMin = 0x1p-110f;
 // 2^127, so none overflows, and what the planes of values under kPlaneMin lose stays under 2^-63.
 constexpr float kPlaneSafe = 0x1p56f;
 
+// Where the result's relative error counts: when no operand is kPlaneBig or more, what the planes of values
+// under kPlaneMin lose of a sum of up to 2^20 products stays under 2^-73, and only results under
+// kPlaneSmall, 2^-25 of which that is, can show it.
+constexpr float kPlaneBig = 0x1p40f, kPlaneSmall = 0x1p-48f;
+
 // the largest of m and the magnitudes of 8 values (v_max3_f32; NaN among them are ignored, or take the
 // place of the two before them)
 __device__ __forceinline__ float abs_max8(const float (&v)[8], float m = 0.f) {
@@ -123,20 +128,24 @@ __device__ __forceinline__ float abs_max8(const float (&v)[8], float m = 0.f) {
   return m;
 }
 
-// true when one of 8 values is non-zero and under kPlaneMin: four v_min3_f32, and a closer look only where
-// a lane of the wave holds such a value or a zero
-__device__ __forceinline__ bool below_planes(const float (&v)[8]) {
+// the smallest magnitude of 8 values
+__device__ __forceinline__ float abs_min8(const float (&v)[8]) {
   float m;
-  asm("v_min3_f32 %0, |%1|, |%2|, |%3|" : "=v"(m) : "v"(v[0]), "v"(v[1]), "v"(v[2]));
-  asm("v_min3_f32 %0, %1, |%2|, |%3|" : "=v"(m) : "v"(m), "v"(v[3]), "v"(v[4]));
-  asm("v_min3_f32 %0, %1, |%2|, |%3|" : "=v"(m) : "v"(m), "v"(v[5]), "v"(v[6]));
-  asm("v_min_f32_e64 %0, %1, |%2|" : "=v"(m) : "v"(m), "v"(v[7]));
-  bool below = false;
-  if (__builtin_amdgcn_ballot_w64(m < kPlaneMin) != 0) {
+  asm("v_min_f32_e64 %0, |%1|, |%2|" : "=v"(m) : "v"(v[0]), "v"(v[1]));
 #pragma unroll
-    for (int e = 0; e < 8; ++e) below |= __builtin_fabsf(v[e]) < kPlaneMin && v[e] != 0.f;
+  for (int e = 2; e < 8; e += 2) asm("v_min3_f32 %0, %1, |%2|, |%3|" : "=v"(m) : "v"(m), "v"(v[e]), "v"(v[e + 1]));
+  return m;
+}
+// true when one of 8 values is non-zero and under kPlaneMin; not so where abs_min8 isn't under it, which a zero
+// also makes it
+__device__ __forceinline__ bool below_planes(const float (&v)[8]) {
+  uint32_t least = ~0u;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const uint32_t t = 2 * __builtin_bit_cast(uint32_t, v[e]) - 1;    // no sign, and a zero becomes the largest
+    least = t < least ? t : least;
   }
-  return below;
+  return least < 2 * __builtin_bit_cast(uint32_t, kPlaneMin) - 1;
 }
 
 // 8 floats as three bf16 planes, v = v0 + v1 + v2 with v0 = bf16(v), v1 = bf16(v - v0),

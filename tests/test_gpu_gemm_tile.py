@@ -121,6 +121,34 @@ def test_tile_gemm_fp32_range(hip, scale):
     _check(_run(x, w, None), _ref(x, w, None), 48)
 
 
+@pytest.mark.parametrize("n,m,o,k", [(520, 128, 128, 72), (200, 64, 64, 40)])
+@pytest.mark.parametrize("xs,ws", [(2.0 ** -107, 1.0), (2.0 ** -112, 1.0), (2.0 ** -120, 1.0), (2.0 ** -126, 1.0),
+                                   (2.0 ** -138, 1.0), (1.0, 2.0 ** -118), (2.0 ** -118, 2.0 ** 60),
+                                   (2.0 ** -118, 2.0 ** 100), (2.0 ** 30, 2.0 ** -118), (2.0 ** -58, 2.0 ** -62)])
+def test_tile_gemm_fp32_small_values(hip, n, m, o, k, xs, ws):
+    """Values below what three bf16 planes carry, alone and beside ordinary ones and zeros: every row and column
+    keeps the fp32 bar.  Subnormal results have steps of 2^-149 besides: 2 k roundings (products and sums) of at most
+    half a step each add 2^-150 sqrt(2 k) in the root mean square."""
+    torch.manual_seed(7)
+    x = torch.randn(n, m, k, device=DEV)
+    w = torch.randn(n, o, k, device=DEV)
+    if xs < ws:
+        x[:, 1::2] *= xs                               # every other row
+        w *= ws
+        x[:, 5] = 0.0
+    else:
+        w[:, ::3] *= ws
+        x *= xs
+        x[:, :, :4] = 0.0
+    got, ref = _run(x, w, None).double(), _ref(x, w, None)
+    for rows, cols in ((slice(1, None, 2), slice(None)), (slice(0, None, 2), slice(None)),
+                       (slice(None), slice(0, None, 3)), (slice(None), slice(1, None, 3))):
+        g, r = got[:, rows, cols], ref[:, rows, cols]
+        bar = 2.0 ** -23 * k ** 0.5 + 2.0 ** -150 * (2 * k * r.numel()) ** 0.5 / r.norm().item()
+        assert ((g - r).norm() / r.norm()).item() <= bar, (rows, cols)
+    assert (got[:, 5] == 0.0).all() or xs >= ws
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("n,m,k,o1,o2", [(40, 200, 96, 128, 256), (100, 65, 40, 64, 128), (3, 20, 64, 32, 64),
                                          (2, 33, 48, 50, 100), (5, 1, 16, 96, 7), (64, 260, 64, 192, 384),
