@@ -236,14 +236,12 @@ void gemm_tile_kernel(GemmParams p) {
       for (int j = 0; j < FN; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) bad |= !(__builtin_fabsf(acc[i][j][e]) <= 3.402823466e38f);
-    bool ask = top >= kPlaneBig;                     // could an operand under kPlaneMin show?
+    float least = INFINITY;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) ask |= __builtin_fabsf(acc[i][j][e]) < kPlaneSmall;
-    if (ask) flags[0] = 1;
+      for (int j = 0; j < FN; ++j) least = abs_min16(acc[i][j], least);
+    if (top >= kPlaneBig || least < kPlaneSmall) flags[0] = 1;     // an operand under kPlaneMin could show
     __syncthreads();
     if (flags[0] != 0) {
       bool below = false;

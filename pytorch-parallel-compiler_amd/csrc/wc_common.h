@@ -136,6 +136,12 @@ __device__ __forceinline__ float abs_min8(const float (&v)[8]) {
   for (int e = 2; e < 8; e += 2) asm("v_min3_f32 %0, %1, |%2|, |%3|" : "=v"(m) : "v"(m), "v"(v[e]), "v"(v[e + 1]));
   return m;
 }
+// the smallest of m and the magnitudes of 16 accumulators
+__device__ __forceinline__ float abs_min16(const f32x16& v, float m) {
+#pragma unroll
+  for (int e = 0; e < 16; e += 2) asm("v_min3_f32 %0, %1, |%2|, |%3|" : "=v"(m) : "v"(m), "v"(v[e]), "v"(v[e + 1]));
+  return m;
+}
 // true when one of 8 values is non-zero and under kPlaneMin; not so where abs_min8 isn't under it, which a zero
 // also makes it
 __device__ __forceinline__ bool below_planes(const float (&v)[8]) {
