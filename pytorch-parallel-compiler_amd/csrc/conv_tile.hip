@@ -9,10 +9,12 @@
 // share a CU, so one's staging runs beside the other's MFMAs.
 //
 // fp32 values are split into three bf16 planes on their way into LDS and multiplied as the six
-// plane products of at most second order (every bit of a normal fp32 value; dropped terms below
-// 2^-26 of a product), which six bf16 MFMAs do in 3/8 of the fp32 MFMA's time.  A wave that ends
-// with an infinity or NaN recomputes its outputs with fp32 multiply-adds from memory, so such
-// inputs give what fp32 arithmetic gives.
+// plane products of at most second order (every bit of an fp32 value from 2^-110 on; dropped terms
+// below 2^-26 of a product), which six bf16 MFMAs do in 3/8 of the fp32 MFMA's time.  A wave that ends
+// with an infinity or NaN recomputes its outputs on the fp32 MFMA from memory, so such inputs give what
+// fp32 arithmetic gives.  So does one of a workgroup that holds operands under 2^-110, which are looked
+// for where they can show: by a result under kPlaneSmall, or an operand of kPlaneBig or more.  (16 models x 8,
+// 64 -> 64, 3x3, 32 x 32: 76 us; a zero filter in every 64: 145 for the look; an infinite or small one: 360.)
 //
 // What bounds it: the MFMAs and, for few taps or channels, staging the input tile (its loads are
 // exposed at every 32-channel chunk but for the other workgroup).  Measured (us; before: the
@@ -50,12 +52,13 @@ __device__ __forceinline__ f32x16 ct_mma(bf16x8 a, bf16x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-// 8 values as PLANES 16-byte rows
+// 8 values as PLANES 16-byte rows; top: the largest fp32 one so far
 template <typename T, int PLANES>
-__device__ __forceinline__ void ct_planes(const T (&v)[8], uint4 (&pl)[PLANES]) {
+__device__ __forceinline__ void ct_planes(const T (&v)[8], uint4 (&pl)[PLANES], float& top) {
   if constexpr (PLANES == 1) {
     __builtin_memcpy(&pl[0], v, 16);
   } else {
+    top = abs_max8(v, top);
     split_planes(v, pl);
   }
 }
@@ -64,7 +67,7 @@ __device__ __forceinline__ void ct_planes(const T (&v)[8], uint4 (&pl)[PLANES]) 
 // 32-channel chunk's rows of all taps, contiguous per output channel, are staged in LDS as they are,
 // and each tap's 8 channels are gathered from there.
 template <typename T, bool RAW>
-__global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && !RAW ? 3 : 2)))
 void conv_tile_kernel(ConvParams p) {
   constexpr int PLANES = sizeof(T) == 4 ? 3 : 1;
   constexpr int WPLANE = 64 * 32;                    // elements of one plane of a tap's weights
@@ -74,6 +77,7 @@ void conv_tile_kernel(ConvParams p) {
   const int xplane = npix * kXPitch;
   uint16_t* const ws = xs + PLANES * xplane;                       // [2][PLANES][64][32]
   T* const raw = reinterpret_cast<T*>(ws + 2 * PLANES * WPLANE);   // RAW: [64][rp]
+  __shared__ int flags[2];                                         // fp32: look at the operands again; compute again
   const int rp = raw_pitch<T>(p);
 
   // ---- tile coordinates ----
@@ -169,9 +173,10 @@ void conv_tile_kernel(ConvParams p) {
         if (dst[u] >= 0) *reinterpret_cast<uint4*>(raw + dst[u]) = v[u];
     }
   };
+  float top = 0.f;
   auto wstash = [&](int buf) {
     uint4 pl[PLANES];
-    ct_planes<T, PLANES>(wreg, pl);
+    ct_planes<T, PLANES>(wreg, pl, top);
 #pragma unroll
     for (int q = 0; q < PLANES; ++q)
       *reinterpret_cast<uint4*>(wdst + (buf * PLANES + q) * WPLANE) = pl[q];
@@ -188,6 +193,7 @@ void conv_tile_kernel(ConvParams p) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) accs[a][i][e] = 0.f;
 
+  if (PLANES == 3 && tid < 2) flags[tid] = 0;
   bool staged = false;
   for (int t = 0; t < p.kd; ++t) {
     const int di = od * p.sd - p.pd + t * p.dd;
@@ -227,7 +233,7 @@ void conv_tile_kernel(ConvParams p) {
           for (int u = 0; u < U; ++u) {
             if (dst[u] < 0) continue;
             uint4 pl[PLANES];
-            ct_planes<T, PLANES>(v[u], pl);
+            ct_planes<T, PLANES>(v[u], pl, top);
 #pragma unroll
             for (int q = 0; q < PLANES; ++q) *reinterpret_cast<uint4*>(xs + q * xplane + dst[u]) = pl[q];
           }
@@ -285,6 +291,28 @@ void conv_tile_kernel(ConvParams p) {
     acc[i] = accs[0][i];
     if constexpr (NACC == 2) acc[i] += accs[1][i];
   }
+  bool bad = false;                                  // fp32: the planes did not carry something
+  if constexpr (PLANES == 3) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) bad |= !(__builtin_fabsf(acc[i][e]) <= 3.402823466e38f);
+    bool small = abs_min16(acc[1], abs_min16(acc[0], INFINITY)) < kPlaneSmall;
+    if (__builtin_amdgcn_ballot_w64(small) != 0) {
+      // of outputs that exist?  The wave's pixels, one a lane; then the lane's own: bit 32 i + 8 q + e
+      const int px = px0 + lane, pr = px / p.tc;
+      const uint64_t mine = __builtin_amdgcn_ballot_w64(pr < p.tr && ho0 + pr < p.ho && wo0 + px - pr * p.tc < p.wo) >>
+                            (4 * hf);
+      small = false;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          small |= __builtin_fabsf(acc[i][e]) < kPlaneSmall && (mine >> (32 * i + 8 * (e >> 2) + (e & 3)) & 1) != 0;
+    }
+    // could an operand under kPlaneMin show?
+    if (top >= kPlaneBig || (small && co0 + cw + l32 < p.co)) flags[0] = 1;
+  }
   // ---- bias and folded BN of the lane's channel, into LDS as [channel][pixel] ----
   const int co = co0 + cw + l32;
   float alpha = 1.f, beta = 0.f;
@@ -300,48 +328,92 @@ void conv_tile_kernel(ConvParams p) {
     }
   }
   __syncthreads();
+  if constexpr (PLANES == 3) {
+    // filters: wrow elements per output channel, tap (t, r, s) of channel c at ((t kh + r) kw + s) wts + c wcs
+    const int wrow = RAW ? p.ci * taps : taps_all * p.ci32, wts = RAW ? 1 : p.ci32, wcs = RAW ? taps : 1;
+    const T* const wall = RAW ? wnb : wb + static_cast<int64_t>(co0) * wrow;
+    if (flags[0] != 0) {
+      bool below = false;
+      const int64_t welems = static_cast<int64_t>(p.co - co0 < 64 ? p.co - co0 : 64) * wrow;
+      for (int64_t e = tid * 8; e < welems; e += kConvThreads * 8) {
+        T v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = e + q < welems ? wall[e + q] : from_f32<T>(0.f);
+        below |= below_planes(v);
+      }
+      for (int t = 0; t < p.kd; ++t) {
+        const int di = od * p.sd - p.pd + t * p.dd;
+        if (di < 0 || di >= p.d) continue;
+        for (int e = tid; e < npix * ((p.ci + 7) / 8); e += kConvThreads) {
+          const int cg = e / npix, rc = e - cg * npix, r = rc / p.ic;
+          const int hi = hi0 + r, wi = wi0 + rc - r * p.ic;
+          const bool in = hi >= 0 && hi < p.h && wi >= 0 && wi < p.w;
+          const T* const xp = xb + static_cast<int64_t>(cg * 8) * p.x_cs + (static_cast<int64_t>(di) * p.h + hi) * p.w + wi;
+          T v[8];
+#pragma unroll
+          for (int q = 0; q < 8; ++q) v[q] = in && cg * 8 + q < p.ci ? xp[q * p.x_cs] : from_f32<T>(0.f);
+          below |= below_planes(v);
+        }
+      }
+      if (below) flags[1] = 1;
+      __syncthreads();
+      bad |= flags[1] != 0;
+    }
+    if (__builtin_amdgcn_ballot_w64(bad) != 0) {
+      // 8 channels of a tap at a time, 4 of each lane half: a step pairs channels c and c + 4.  A padding pixel is
+      // a zero that meets the weight: an infinite weight gives NaN there.
+      const T* const wl = wall + static_cast<int64_t>(co0 + cw + l32 < p.co ? cw + l32 : p.co - 1 - co0) * wrow;
+      int prow[2], pcol[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int px = px0 + i * 32 + l32, pr = px / p.tc;
+        prow[i] = pr < p.tr ? hi0 + pr * p.sh : hi0; // pixels past the tile repeat its first
+        pcol[i] = pr < p.tr ? wi0 + (px - pr * p.tc) * p.sw : wi0;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
+      }
+      for (int t = 0; t < p.kd; ++t) {
+        const int di = od * p.sd - p.pd + t * p.dd;
+        if (di < 0 || di >= p.d) continue;
+        for (int r = 0; r < p.kh; ++r)
+          for (int s = 0; s < p.kw; ++s) {
+            const T* xp[2];
+            bool in[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+              const int hi = prow[i] + r * p.dh, wi = pcol[i] + s * p.dw;
+              in[i] = hi >= 0 && hi < p.h && wi >= 0 && wi < p.w;
+              xp[i] = xb + (static_cast<int64_t>(di) * p.h + hi) * p.w + wi;
+            }
+            const T* const wp = wl + static_cast<int64_t>((t * p.kh + r) * p.kw + s) * wts;
+            for (int c0 = 4 * hf; c0 - 4 * hf < p.ci; c0 += 8)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const int c = c0 + e;
+                const float wv = c < p.ci ? to_f32(wp[c * wcs]) : 0.f;
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                  const float xv = c < p.ci && in[i] ? to_f32(xp[i][c * p.x_cs]) : 0.f;
+                  acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(xv, wv, acc[i], 0, 0, 0);
+                }
+              }
+          }
+      }
+    }
+  }
   constexpr int CPITCH = kTPix + 8;
   T* const cs = reinterpret_cast<T*>(smem4);
-  bool bad = false;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       T o[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float v = acc[i][4 * q + e];
-        bad |= !(__builtin_fabsf(v) <= 3.402823466e38f);
-        o[e] = from_f32<T>(v * alpha + beta);
-      }
+      for (int e = 0; e < 4; ++e) o[e] = from_f32<T>(acc[i][4 * q + e] * alpha + beta);
       // lane: channel l32, pixels 8 q + 4 hf + (0 .. 3) of the fragment
       __builtin_memcpy(__builtin_assume_aligned(cs + (cw + l32) * CPITCH + px0 + i * 32 + 8 * q + 4 * hf, 4 * sizeof(T)),
                        o, sizeof(o));
     }
-  if (PLANES == 3 && __builtin_amdgcn_ballot_w64(bad) != 0 && co < p.co) {
-    // infinities and NaN: the lane's outputs again, in fp32 from memory
-    const T* const wr = RAW ? wnb + static_cast<int64_t>(co - co0) * p.ci * taps
-                            : wb + static_cast<int64_t>(co) * taps_all * p.ci32;
-    const int wcs = RAW ? taps : 1;                  // from one input channel to the next
-    for (int e = 0; e < 32; ++e) {
-      const int px = px0 + (e >> 4) * 32 + ((e & 15) >> 2) * 8 + 4 * hf + (e & 3);
-      const int pr = px / p.tc, pc = px - (px / p.tc) * p.tc;
-      if (pr >= p.tr || ho0 + pr >= p.ho || wo0 + pc >= p.wo) continue;
-      float v = 0.f;
-      for (int t = 0; t < p.kd; ++t)
-        for (int r = 0; r < p.kh; ++r)
-          for (int s = 0; s < p.kw; ++s) {
-            const int di = od * p.sd - p.pd + t * p.dd, hi = hi0 + pr * p.sh + r * p.dh, wi = wi0 + pc * p.sw + s * p.dw;
-            if (di < 0 || di >= p.d) continue;
-            // a padding pixel is a zero that meets the weight: an infinite weight gives NaN there
-            const bool in = hi >= 0 && hi < p.h && wi >= 0 && wi < p.w;
-            const T* xp = xb + (static_cast<int64_t>(di) * p.h + (in ? hi : 0)) * p.w + (in ? wi : 0);
-            const T* wp = wr + static_cast<int64_t>((t * p.kh + r) * p.kw + s) * (RAW ? 1 : p.ci32);
-            for (int c = 0; c < p.ci; ++c) v += (in ? to_f32(xp[c * p.x_cs]) : 0.f) * to_f32(wp[c * wcs]);
-          }
-      cs[(cw + l32) * CPITCH + px] = from_f32<T>(v * alpha + beta);
-    }
-  }
   __syncthreads();
   conv_store<T, kTPix>(p, cs, mdl, bb, ho0, wo0, co0, od);
 }
@@ -366,7 +438,7 @@ bool tile_plan(ConvParams& p, size_t& lds) {
       const double tiles = static_cast<double>(cdiv(p.ho, tr)) * static_cast<double>(cdiv(p.wo, tc));
       // staging a pixel costs about as much as the MFMAs of 4 / taps output pixels
       double cost = tiles * (kTPix + 4.0 * static_cast<double>(ir * ic) / (p.kh * p.kw));
-      if (bytes(ir, ic) > 80 * 1024) cost *= 1.5;
+      if (bytes(ir, ic) > 80 * 1024 - 16) cost *= 1.5;     // 16: the kernel's flags
       if (best < 0.0 || cost < best) {
         best = cost;
         p.tr = tr;

@@ -136,6 +136,38 @@ def test_conv_tile_fp32_infinite_weight_meets_padding(hip):
     assert torch.equal(torch.isinf(got), torch.isinf(f))
 
 
+@pytest.mark.parametrize("ci,co,hw", [(20, 40, 17), (40, 70, 30), (16, 24, 9)])
+@pytest.mark.parametrize("xs,ws", [(2.0 ** -107, 1.0), (2.0 ** -112, 1.0), (2.0 ** -120, 1.0), (2.0 ** -138, 1.0),
+                                   (1.0, 2.0 ** -118), (2.0 ** -118, 2.0 ** 60), (2.0 ** -58, 2.0 ** -62)])
+def test_conv_tile_fp32_small_values(hip, ci, co, hw, xs, ws):
+    """Values below what three bf16 planes carry in one image or in some filters, beside ordinary ones and zeros:
+    every image and filter keeps the fp32 bar.  Subnormal results have steps of 2^-149 besides: 2 K roundings of
+    at most half a step each add 2^-150 sqrt(2 K) in the root mean square."""
+    from wide_compiler import _hip
+    torch.manual_seed(6)
+    n, b = 3, 2
+    x = torch.randn(n, b, ci, hw, hw, device=DEV)
+    w = torch.randn(n * co, ci, 3, 3, device=DEV)
+    if xs < ws:
+        x[:, 1] *= xs
+        w *= ws
+        x[:, 1, 3] = 0.0
+    else:
+        w[::3] *= ws
+        x *= xs
+    y = torch.full((n, b, co, hw, hw), float("nan"), device=DEV)
+    _hip.conv2d(x=x, weight=w, n=n, c_in=ci, c_out=co, kernel=(3, 3), stride=(1, 1), padding=(1, 1), dilation=(1, 1),
+                y=y, bias=None)
+    got = y.double().cpu().reshape(n, b, co, -1)
+    ref = torch.stack([nn.functional.conv2d(x[q].double().cpu(), w[q * co:(q + 1) * co].double().cpu(), padding=1)
+                       for q in range(n)]).reshape(n, b, co, -1)
+    for image in range(b):
+        for at in range(3):
+            g, r = (t.reshape(n, b, co, -1)[:, image].reshape(n * co, -1)[at::3] for t in (got, ref))
+            bar = 2.0 ** -23 * (9 * ci) ** 0.5 + 2.0 ** -150 * (18 * ci * r.numel()) ** 0.5 / r.norm().item()
+            assert ((g - r).norm() / r.norm()).item() <= bar, (image, at)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("n,b,ci,co,h,w,kh,kw,stride,pad", [
     (2, 3, 3, 40, 9, 12, 3, 3, 1, 1),        # rows of 27 values; channels past a tile's first 32
