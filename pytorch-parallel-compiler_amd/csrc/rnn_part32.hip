@@ -5,7 +5,7 @@
 // so P = H / (16 TPW) workgroups share a unit of (model, up to 16 batch rows), one per compute
 // unit, for all T steps.  A workgroup owns 16 TPW hidden units and holds the rows of W_hh of
 // their gates in registers for the whole sequence, split into three bf16 planes
-// (v = v0 + v1 + v2 exactly; the products of at most second order in fp32, as in the tile GEMM).
+// (v = v0 + v1 + v2; the products of at most second order in fp32, as in the tile GEMM).
 //
 // Per step: gates = h_{t-1} W_hh^T as 16x16x32 MFMAs (A = W_hh planes, B = h planes from LDS),
 // the cell update in registers (the fp32 state never leaves the chip), h_t into its place in the
@@ -26,8 +26,9 @@
 // are invalid.  The host launches the grid cooperatively (all workgroups co-resident, or the
 // launch fails); a captured stream takes the one-launch-per-step kernel instead.
 //
-// Infinities: a workgroup whose W_hh rows, or a step whose h, hold one (or a value that rounds to
-// one in bf16) computes its gates with fp32 multiply-adds from memory instead.
+// What the planes do not carry: a workgroup whose W_hh rows, or a step whose h, hold a value of 2^56 or more
+// (kPlaneSafe) or an infinity computes its gates with fp32 multiply-adds from memory instead.  Below it no gate
+// sum overflows, and what the planes lose of a value under 2^-110 stays 2^-60 of a gate's range.
 //
 // Bound by the step's serial chain: MFMAs (and the LDS reads that feed them), the store, flag and
 // load latencies of the exchange.  Measured (us; before: one launch per step, streaming W_hh):
@@ -69,16 +70,16 @@ __device__ __forceinline__ void sync_store(int* p, int v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// 8 floats as planes; true when one is infinite or may round to it (NaN stays NaN in the planes)
+// 8 floats as planes; true when one is kPlaneSafe or more (NaN stays NaN in the planes)
 __device__ __forceinline__ bool split8(const float (&v)[8], bf16x8 (&pl)[3]) {
-  bool bad = false;
+  bool big = false;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) bad |= __builtin_fabsf(v[e]) > kPlaneMax;
+  for (int e = 0; e < 8; ++e) big |= __builtin_fabsf(v[e]) >= kPlaneSafe;
   uint4 u[3];
   split_planes(v, u);
 #pragma unroll
   for (int q = 0; q < 3; ++q) pl[q] = __builtin_bit_cast(bf16x8, u[q]);
-  return bad;
+  return big;
 }
 
 template <int KS, int TPW, int CELL>

@@ -108,8 +108,8 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
 
-// The range of values that split_planes (below) carries.
-constexpr float kPlaneMax = 3.38e38f, kPlaneMin = 0x1p-110f;
+// The smallest value that split_planes (below) carries with all its bits.
+constexpr float kPlaneMin = 0x1p-110f;
 // Below kPlaneSafe the planes of a dot product's operands need no further look where only the sum's
 // absolute error counts (a score, a gate): products and their sums of up to 2^14 terms stay under
 // 2^127, so none overflows, and what the planes of values under kPlaneMin lose stays under 2^-63.
@@ -120,9 +120,17 @@ constexpr float kPlaneSafe = 0x1p56f;
 // kPlaneSmall, 2^-25 of which that is, can show it.
 constexpr float kPlaneBig = 0x1p40f, kPlaneSmall = 0x1p-48f;
 
-// the largest of m and the magnitudes of 8 values (v_max3_f32; NaN among them are ignored, or take the
-// place of the two before them)
-__device__ __forceinline__ float abs_max8(const float (&v)[8], float m = 0.f) {
+// The largest magnitude of 8 values (v_max3_f32; NaN among them are ignored, or take the place of those before
+// them), and of them and m.
+__device__ __forceinline__ float abs_max8(const float (&v)[8]) {
+  float a, b;
+  asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(a) : "v"(v[0]), "v"(v[1]), "v"(v[2]));
+  asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(b) : "v"(v[3]), "v"(v[4]), "v"(v[5]));
+  asm("v_max3_f32 %0, %1, %2, |%3|" : "=v"(a) : "v"(a), "v"(b), "v"(v[6]));
+  asm("v_max_f32_e64 %0, %1, |%2|" : "=v"(a) : "v"(a), "v"(v[7]));
+  return a;
+}
+__device__ __forceinline__ float abs_max8(const float (&v)[8], float m) {
 #pragma unroll
   for (int e = 0; e < 8; e += 2) asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(m) : "v"(m), "v"(v[e]), "v"(v[e + 1]));
   return m;
@@ -156,8 +164,8 @@ __device__ __forceinline__ bool below_planes(const float (&v)[8]) {
 
 // 8 floats as three bf16 planes, v = v0 + v1 + v2 with v0 = bf16(v), v1 = bf16(v - v0),
 // v2 = v - v0 - v1: every bit of an fp32 value from kPlaneMin on.  Below it bits fall under 2^-133, the
-// smallest bf16, and up to 2^-134 is lost.  Infinities, NaN and values above kPlaneMax (they may
-// round to infinity) leave NaN in the planes.
+// smallest bf16, and up to 2^-134 is lost.  Infinities, NaN and values that round to infinity (from
+// 3.39e38 on) leave NaN in the planes.
 __device__ __forceinline__ void split_planes(const float (&v)[8], uint4 (&pl)[3]) {
   float f[8];
 #pragma unroll

@@ -163,3 +163,49 @@ def test_part32_infinite_weights_and_states(hip, kind):
     assert torch.equal(torch.isnan(out.cpu()), torch.isnan(ref))
     keep = ~torch.isnan(ref)
     assert (out.cpu().double()[keep] - ref[keep]).abs().max().item() <= 1e-5
+
+
+@pytest.mark.parametrize("kind", ["lstm", "gru"])
+@pytest.mark.parametrize("hv,wv", [(3.01e20, 3.01e20), (1.003e3, 3e38), (2.0 ** 90, 2.0 ** 60)])
+def test_part32_gate_sums_that_overflow(hip, kind, hv, wv):
+    """A finite h0 and finite weights whose gate sums overflow saturate the gate, as in fp32: the LSTM's first gate
+    of every fourth unit (0) and its third (-1), and the GRU's update gate of every unit (h_1 = n)."""
+    torch.manual_seed(9)
+    n, b, t, i, h = 2, 3, 12, 8, 256
+    mods = _mods(kind, n, i, h)
+    with torch.no_grad():
+        for m in mods:
+            m.weight_hh_l0 /= hv
+            if kind == "lstm":
+                m.weight_hh_l0[0:h:4] = -wv
+                m.weight_hh_l0[2 * h:3 * h:3] = -wv
+            else:
+                m.weight_hh_l0[h:2 * h] = -wv
+    states = [torch.randn(n, b, h) * 0.5 for _ in range(2 if kind == "lstm" else 1)]
+    states[0][:] = hv
+    wide = _wide(kind, mods)
+    x = torch.randn(n, b, t, i)
+    out, _ = _run(wide, x, states)
+    hip.rnn_sync_check(block=True)
+    ref, _ = _ref(mods, x, states)
+    assert not torch.isnan(out).any()
+    assert rel_err(out[:, :, 0], ref[:, :, 0]) <= TOL_F32
+
+
+@pytest.mark.parametrize("kind", ["lstm", "gru"])
+def test_part32_states_and_weights_far_apart(hip, kind):
+    """Subnormal-range states on weights near the top of the range: gates of order one keep the fp32 bar."""
+    torch.manual_seed(10)
+    n, b, t, i, h = 2, 3, 12, 8, 256
+    mods = _mods(kind, n, i, h)
+    with torch.no_grad():
+        for m in mods:
+            m.weight_hh_l0[:, 17] = torch.randn(m.weight_hh_l0.shape[0]) * 2.0 ** 122
+    states = [torch.randn(n, b, h) * 0.5 for _ in range(2 if kind == "lstm" else 1)]
+    states[0][:, :, 17] = torch.randn(n, b) * 2.0 ** -122
+    wide = _wide(kind, mods)
+    x = torch.randn(n, b, t, i)
+    out, _ = _run(wide, x, states)
+    hip.rnn_sync_check(block=True)
+    ref, _ = _ref(mods, x, states)
+    assert rel_err(out[:, :, 0], ref[:, :, 0]) <= TOL_F32
