@@ -209,7 +209,7 @@ typedef struct wc_rnn_args {
                                 up, and the library never clears it (so it also collects
                                 the verdicts of graph replays until the caller reads and
                                 clears it).  NULL: the workspace's own status word
-                                (wc_rnn_status_offset), zeroed by every input projection. */
+                                (wc_rnn_status_offset), zeroed by every forward. */
 } wc_rnn_args;
 
 /* Bytes of workspace wc_rnn_forward needs for these sizes on the current device.
@@ -221,9 +221,9 @@ typedef struct wc_rnn_args {
 int64_t wc_rnn_workspace_bytes(const wc_rnn_args* args);
 
 /* Byte offset in the workspace of the int32 status word of the partitioned plan, or
- * -1 when these sizes use another plan.  wc_rnn_input_projection (fp32: wc_rnn_recurrence)
- * zeroes it; the recurrence sets it to 1 if a cross-workgroup wait timed out, in which
- * case out / h_n / c_n are invalid. */
+ * -1 when these sizes use another plan.  wc_rnn_input_projection (fp32: wc_rnn_recurrence,
+ * captured or not) zeroes it; the recurrence sets it to 1 if a cross-workgroup wait timed out,
+ * in which case out / h_n / c_n are invalid.  It holds when the recurrence has finished. */
 int64_t wc_rnn_status_offset(const wc_rnn_args* args);
 
 /* Poll rounds after which a wait of the partitioned LSTM gives up, for launches made
@@ -259,7 +259,7 @@ int32_t wc_rnn_input_projection(const wc_rnn_args* args, void* stream);
  *  - Partitioned plan in fp32 (LSTM or GRU, hidden above 128 up to 384, a multiple of 32,
  *    16-byte aligned w_hh / h0 / out, long enough sequences): hidden/16 or hidden/32
  *    workgroups per unit, exchanging h_t through the output; cooperative launches.  A
- *    captured stream takes the next form instead.
+ *    captured stream takes the next form instead (the status word then reads 0).
  *  - Otherwise one launch per step (an MFMA gate GEMM fused with the cell update;
  *    hidden % 32 == 0). */
 int32_t wc_rnn_recurrence(const wc_rnn_args* args, void* stream);

@@ -739,6 +739,25 @@ static int32_t persistent_recurrence(const wc_rnn_args* a, RnnParams p, int gate
   return launch_rec<bf16, WC_CELL_LSTM>(p, grid, block, lds, st);
 }
 
+// The time loop without cross-workgroup waits: the persistent kernel, or one launch per step.
+static int32_t unshared_recurrence(const wc_rnn_args* a, RnnParams& p, int gates, hipStream_t st) {
+  if (rnn_plan(gates, p.hid, p)) return persistent_recurrence(a, p, gates, st);
+  // W_hh of one model does not fit a workgroup's registers: one launch per step
+  const int es = dtype_size(a->dtype);
+  WC_REQUIRE(aligned(a->w_hh, 16) && ubytes(p.hid, es) % 16 == 0 && p.hid % 32 == 0 &&
+                 (!a->h0 || aligned(a->h0, 16)) && aligned(a->out, 16),
+             WC_ERR_ALIGN, "wc_rnn_recurrence: hidden=%d needs hidden %% 32 == 0 and 16-byte aligned "
+             "W_hh / h0 / out for the streamed recurrence", p.hid);
+  if (a->dtype == WC_F32)
+    return a->cell == WC_CELL_GRU ? streamed_recurrence<float, WC_CELL_GRU>(a, p, st)
+                                  : streamed_recurrence<float, WC_CELL_LSTM>(a, p, st);
+  if (a->dtype == WC_F16)
+    return a->cell == WC_CELL_GRU ? streamed_recurrence<f16, WC_CELL_GRU>(a, p, st)
+                                  : streamed_recurrence<f16, WC_CELL_LSTM>(a, p, st);
+  return a->cell == WC_CELL_GRU ? streamed_recurrence<bf16, WC_CELL_GRU>(a, p, st)
+                                : streamed_recurrence<bf16, WC_CELL_LSTM>(a, p, st);
+}
+
 extern "C" int32_t wc_rnn_recurrence(const wc_rnn_args* a, void* stream) {
   clear_error();
   RnnParams p;
@@ -753,25 +772,11 @@ extern "C" int32_t wc_rnn_recurrence(const wc_rnn_args* a, void* stream) {
     if (hipStreamIsCapturing(as_stream(stream), &cap) != hipSuccess)
       return set_error(WC_ERR_ARG, "wc_rnn_recurrence: stream capture status unavailable");
     if (cap == hipStreamCaptureStatusNone) return part32_recurrence(a, as_stream(stream));
+    // captured: no waits that could give up, but the workspace's status word lies in the cell state
+    rc = unshared_recurrence(a, p, gates, as_stream(stream));
+    return rc || a->status ? rc : part32_clear_status(a, as_stream(stream));
   }
-  if (!rnn_plan(gates, p.hid, p)) {
-    // W_hh of one model does not fit a workgroup's registers: one launch per step
-    const int es = dtype_size(a->dtype);
-    WC_REQUIRE(aligned(a->w_hh, 16) && ubytes(p.hid, es) % 16 == 0 && p.hid % 32 == 0 &&
-                   (!a->h0 || aligned(a->h0, 16)) && aligned(a->out, 16),
-               WC_ERR_ALIGN, "wc_rnn_recurrence: hidden=%d needs hidden %% 32 == 0 and 16-byte aligned "
-               "W_hh / h0 / out for the streamed recurrence", p.hid);
-    hipStream_t st = as_stream(stream);
-    if (a->dtype == WC_F32)
-      return a->cell == WC_CELL_GRU ? streamed_recurrence<float, WC_CELL_GRU>(a, p, st)
-                                    : streamed_recurrence<float, WC_CELL_LSTM>(a, p, st);
-    if (a->dtype == WC_F16)
-      return a->cell == WC_CELL_GRU ? streamed_recurrence<f16, WC_CELL_GRU>(a, p, st)
-                                    : streamed_recurrence<f16, WC_CELL_LSTM>(a, p, st);
-    return a->cell == WC_CELL_GRU ? streamed_recurrence<bf16, WC_CELL_GRU>(a, p, st)
-                                  : streamed_recurrence<bf16, WC_CELL_LSTM>(a, p, st);
-  }
-  return persistent_recurrence(a, p, gates, as_stream(stream));
+  return unshared_recurrence(a, p, gates, as_stream(stream));
 }
 
 extern "C" int32_t wc_rnn_forward(const wc_rnn_args* a, void* stream) {

@@ -458,6 +458,12 @@ bool part32_plan(const wc_rnn_args* a) {
 
 int64_t part32_status_offset(const wc_rnn_args* a) { return p32_sync_offset(a) + kSyncStatus * 4; }
 
+int32_t part32_clear_status(const wc_rnn_args* a, hipStream_t st) {
+  part32_zero_kernel<<<dim3(1), dim3(64), 0, st>>>(
+      reinterpret_cast<int*>(static_cast<char*>(a->workspace) + part32_status_offset(a)), 1);
+  return check_launch("wc_rnn_recurrence(status)");
+}
+
 int32_t part32_recurrence(const wc_rnn_args* a, hipStream_t st) {
   const int cus = device_cu_count();
   const int tpw = p32_tpw(a, cus);

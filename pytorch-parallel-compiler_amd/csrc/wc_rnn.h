@@ -42,6 +42,9 @@ bool part_cooperative();
 // in the workspace that the one-launch-per-step kernel sizes for its cell state
 bool part32_plan(const wc_rnn_args* a);
 int64_t part32_status_offset(const wc_rnn_args* a);
+// after another kernel has run these sizes: the workspace's status word, which lies in that kernel's cell
+// state, reads 0
+int32_t part32_clear_status(const wc_rnn_args* a, hipStream_t st);
 int32_t part32_recurrence(const wc_rnn_args* a, hipStream_t st);
 
 }  // namespace wc

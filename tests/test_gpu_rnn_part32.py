@@ -209,3 +209,43 @@ def test_part32_states_and_weights_far_apart(hip, kind):
     hip.rnn_sync_check(block=True)
     ref, _ = _ref(mods, x, states)
     assert rel_err(out[:, :, 0], ref[:, :, 0]) <= TOL_F32
+
+
+@pytest.mark.parametrize("kind", ["lstm", "gru"])
+def test_part32_status_word_after_replays(hip, kind):
+    """Without a status word of the caller's the workspace's own one reads 0 after a clean forward, also a
+    captured one, which runs another kernel and finds the workspace in any state."""
+    import ctypes
+    torch.manual_seed(11)
+    n, b, t, i, h = 4, 18, 14, 32, 256
+    wide = _wide(kind, _mods(kind, n, i, h))
+    x = torch.randn(n, b, t, i, device=DEV)
+    out = torch.empty(n, b, t, h, device=DEV)
+    a, ws = hip.rnn_args(cell=hip.CELL_LSTM if kind == "lstm" else hip.CELL_GRU, x=x, w_ih=wide.weight_ih.detach(),
+                         w_hh=wide.weight_hh.detach(), b_ih=wide.bias_ih.detach(), b_hh=wide.bias_hh.detach(),
+                         h0=None, c0=None, out=out, h_n=None, c_n=None)
+    at = hip.lib().wc_rnn_status_offset(ctypes.byref(a))
+    assert 0 <= at <= ws.numel() - 4
+    word = ws[at:at + 4].view(torch.int32)
+
+    def both():
+        hip.rnn_phase(a, "input_projection", x)
+        hip.rnn_phase(a, "recurrence", x)
+
+    ws.fill_(255)
+    both()
+    torch.cuda.synchronize()
+    assert word.item() == 0
+    with torch.no_grad():
+        ref = wide(x)[0]
+    assert rel_err(out, ref) <= TOL_F32
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        both()
+    for _ in range(3):
+        ws.fill_(255)
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert word.item() == 0
+        assert rel_err(out, ref) <= TOL_F32
