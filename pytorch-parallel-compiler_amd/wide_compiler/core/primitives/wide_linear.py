@@ -174,9 +174,14 @@ class WideMLP2(nn.Module):
         return p1["weight"], p1.get("bias"), p2["weight"], p2.get("bias")
 
     def _entry(self, x: Tensor) -> Optional[str]:
-        """The entry point that runs x ([N, ..., in]) as one launch; None: two GEMMs."""
-        return _hip.mlp2_entry(self.first.weight.dtype, self.n, max(math.prod(x.shape[1:-1]), 1), self.in_features,
-                               self.hidden, self.out_features)
+        """The entry point that runs x ([N, ..., in]) as one launch; None: two GEMMs.  The answer for the last
+        (dtype, rows) is kept: it depends on nothing else, and asking the library costs 3 us."""
+        form = (self.first._parameters["weight"].dtype, max(math.prod(x.shape[1:-1]), 1))
+        route = self.__dict__.get("_route")
+        if route is None or route[0] != form:
+            route = self.__dict__["_route"] = (form, _hip.mlp2_entry(form[0], self.n, form[1], self.in_features,
+                                                                     self.hidden, self.out_features))
+        return route[1]
 
     def split(self, x: Tensor) -> Optional[Tensor]:
         """Where x is to run as two GEMMs, the first one's output; else None (nothing run).  A caller

@@ -215,3 +215,22 @@ def test_torch_compile_sees_the_traced_forward_as_one_operator():
     ops = [nd.target for nd in graphs[0].graph.nodes if nd.op == "call_function"]
     assert torch.ops.wide_compiler.module_call.default in ops or torch.ops.wide_compiler.module_call in ops
     assert len([o for o in ops if "module_call" in str(o)]) == 1
+
+
+def test_linear_chain_asks_for_its_route_once_per_form(monkeypatch):
+    """Whether a Linear-Linear chain runs as one launch depends on its dtype and sizes only: a second forward
+    of the same form does not ask the library again, one of another form does."""
+    from wide_compiler import _hip
+    from wide_compiler.core.primitives.wide_linear import WideLinear, WideMLP2
+    asked = []
+    monkeypatch.setattr(_hip, "mlp2_entry", lambda *a: asked.append(a))
+    chain = WideMLP2(WideLinear(2, 8, 16), WideLinear(2, 16, 4), True)
+    for _ in range(3):
+        assert chain._entry(torch.zeros(2, 5, 8)) is None
+    assert len(asked) == 1
+    chain._entry(torch.zeros(2, 6, 8))
+    chain._entry(torch.zeros(2, 3, 2, 8))                    # also 6 rows
+    assert len(asked) == 2 and asked[1][2] == 6
+    chain.to(torch.bfloat16)
+    chain._entry(torch.zeros(2, 6, 8))
+    assert len(asked) == 3 and asked[2][0] == torch.bfloat16
