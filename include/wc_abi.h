@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define WC_ABI_VERSION 6
+#define WC_ABI_VERSION 7
 
 /* element types */
 enum {

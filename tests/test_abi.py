@@ -205,3 +205,15 @@ def test_self_attention_arg_checks(hip):
         setattr(a, field, old)
     a.n = 0
     assert lib.wc_self_attention(ctypes.byref(a), None) == 0
+
+
+# a digest of include/wc_abi.h without comments, per version
+DECLARATIONS = {7: "81bc311c918d84aa037bc7f4e77840e169a1681ecf91b2dcbc77c5d7fa877232"}
+
+
+def test_every_change_of_the_header_has_a_version_of_its_own(hip):
+    """A library and a binding of one version agree on every declaration: what changes the header's entry points,
+    structs or constants takes the next version, and its digest is added here."""
+    import hashlib
+    text = re.sub(r"/\*.*?\*/", "", open(HEADER).read(), flags=re.S)
+    assert DECLARATIONS.get(hip.ABI_VERSION) == hashlib.sha256(" ".join(text.split()).encode()).hexdigest()
