@@ -2,7 +2,10 @@
  *   int32_t entry(const args*, void* stream)
  * by address.  A ctypes call costs about 3 us on the host, most of a small wide forward's
  * dispatch time; this call costs a fraction of that.  The caller passes the entry point's
- * address, the address of its filled argument block and the stream handle as integers. */
+ * address, the address of its filled argument block and the stream handle as integers.  Like a
+ * ctypes call, the entry points run without the interpreter lock (a launch can wait in the runtime
+ * when its queue is full); call2 alone holds it, because its block belongs to the module and
+ * another thread's forward may fill it next. */
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <stdint.h>
@@ -41,7 +44,12 @@ static PyObject* callb(PyObject* self, PyObject* const* args, Py_ssize_t nargs) 
     PyErr_SetString(PyExc_ValueError, "callb: null entry point");
     return NULL;
   }
-  return PyLong_FromLong((long)((wc_entry2)fn)(PyBytes_AS_STRING(args[1]), s));
+  const void* block = PyBytes_AS_STRING(args[1]);      /* the caller's reference outlives the call */
+  int32_t rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = ((wc_entry2)fn)(block, s);
+  Py_END_ALLOW_THREADS
+  return PyLong_FromLong((long)rc);
 }
 
 typedef int32_t (*wc_layernorm_t)(const void*, int64_t, int64_t, const void*, const void*, void*, int64_t, int64_t,
@@ -69,8 +77,12 @@ static PyObject* layernorm(PyObject* self, PyObject* const* a, Py_ssize_t nargs)
     PyErr_SetString(PyExc_ValueError, "layernorm: null entry point");
     return NULL;
   }
-  return PyLong_FromLong((long)((wc_layernorm_t)fn)(x, i[0], i[1], g, b, y, i[2], i[3], i[4], i[5], i[6], (float)eps,
-                                                    (int32_t)dt, (int32_t)pdt, st));
+  int32_t rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = ((wc_layernorm_t)fn)(x, i[0], i[1], g, b, y, i[2], i[3], i[4], i[5], i[6], (float)eps, (int32_t)dt,
+                            (int32_t)pdt, st);
+  Py_END_ALLOW_THREADS
+  return PyLong_FromLong((long)rc);
 }
 
 typedef int32_t (*wc_conv_pack_t)(const void*, int64_t, int64_t, int64_t, int64_t, int64_t, int32_t, void*, void*);
@@ -92,7 +104,11 @@ static PyObject* conv_pack(PyObject* self, PyObject* const* a, Py_ssize_t nargs)
     PyErr_SetString(PyExc_ValueError, "conv_pack: null entry point");
     return NULL;
   }
-  return PyLong_FromLong((long)((wc_conv_pack_t)fn)(w, i[0], i[1], i[2], i[3], i[4], (int32_t)dt, out, st));
+  int32_t rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = ((wc_conv_pack_t)fn)(w, i[0], i[1], i[2], i[3], i[4], (int32_t)dt, out, st);
+  Py_END_ALLOW_THREADS
+  return PyLong_FromLong((long)rc);
 }
 
 static PyMethodDef methods[] = {

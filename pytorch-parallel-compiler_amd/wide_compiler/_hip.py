@@ -606,12 +606,7 @@ def rnn_forward(**kw) -> None:
     rnn_sync_check()
     a, ws = rnn_args(**kw)
     word = _part_status(a, kw["x"])
-    if _wc_launch is not None:
-        rc = _wc_launch.call2(_entries.get("wc_rnn_forward") or entry_address("wc_rnn_forward"), ctypes.addressof(a),
-                              stream_of(kw["x"]))
-    else:
-        rc = lib().wc_rnn_forward(ctypes.byref(a), stream_of(kw["x"]))
-    _check(rc, "wc_rnn_forward")
+    _launch("wc_rnn_forward", _RnnArgs, bytes(a), stream_of(kw["x"]))
     if word is not None:
         _rnn_watch(word)
 

@@ -217,3 +217,28 @@ def test_every_change_of_the_header_has_a_version_of_its_own(hip):
     import hashlib
     text = re.sub(r"/\*.*?\*/", "", open(HEADER).read(), flags=re.S)
     assert DECLARATIONS.get(hip.ABI_VERSION) == hashlib.sha256(" ".join(text.split()).encode()).hexdigest()
+
+
+def test_launches_do_not_hold_the_interpreter_lock():
+    """A launch that waits in the runtime (a full queue) leaves other Python threads running, as a ctypes call
+    does.  The entry point here is libc's sem_timedwait(semaphore, deadline): it returns 0 once another
+    thread has posted the semaphore, -1 when that thread did not get to run within the deadline."""
+    import threading
+    import time
+    from wide_compiler import _wc_launch
+    libc = ctypes.CDLL(None, use_errno=True)
+    sem = bytes(64)
+    at = ctypes.cast(ctypes.c_char_p(sem), ctypes.c_void_p).value
+    assert libc.sem_init(ctypes.c_void_p(at), 0, 0) == 0
+    wait = ctypes.cast(libc.sem_timedwait, ctypes.c_void_p).value
+
+    def post():
+        time.sleep(0.05)
+        libc.sem_post(ctypes.c_void_p(at))
+
+    deadline = (ctypes.c_long * 2)(int(time.time()) + 3, 0)
+    t = threading.Thread(target=post)
+    t.start()
+    rc = _wc_launch.callb(wait, sem, ctypes.addressof(deadline))
+    t.join()
+    assert rc == 0
