@@ -1176,20 +1176,28 @@ extern "C" int32_t wc_attention(const wc_attn_args* a, void* stream) {
   }
   p.dh = (int)a->head_dim;
   p.oc0 = 0;
-  if (al && !p.mask && !p.causal && a->dtype == WC_BF16 && a->head_dim == 32 && a->sq > 256) {
+  if (al && !p.mask && !p.causal && a->dtype == WC_BF16 && a->head_dim == 32) {
     // resident-KV kernel: K and V of one head in LDS, 8-byte aligned output rows.  It folds the
-    // scale into Q and so needs one VALU instruction less per score than the streaming kernel,
-    // but stages all keys before it starts: worth it while its 512-query workgroups cover the
-    // CUs in one round or share a CU two at a time (128 x 8 heads of 512 tokens: 60.4 us against
-    // 69.4; 16 x 8 of 1000: 32.3 against 35.4; 16 x 8 of 512: 17.9 against 13.8; 64 x 8 of 700,
-    // four rounds of one workgroup per CU: 89 against 67)
+    // scale into Q and so needs one VALU instruction less per score than the streaming kernel, but
+    // stages all keys before it starts, in workgroups of 512 queries, so it wants its rounds of one
+    // workgroup per CU full.  `filled`: the share of the rounds' query places that hold a query.  Measured
+    // (us, resident / streaming; heads x tokens):
+    //   one round:                      128 x 1000 (filled 0.98) 32.3 / 36.5   112 x 800 (0.68) 25.5 / 29.5
+    //                                   128 x 600 (0.59) 21.7 / 20.1           96 x 600 (0.44) 20.9 / 16.0
+    //   more, two workgroups in a CU's  512 x 512 (1.00) 34.3 / 37.5           448 x 400 (0.68) 27.3 / 29.8
+    //   LDS (up to 80 KB):              320 x 512 (0.63) 30.3 / 29.5           320 x 400 (0.49) 25.1 / 22.5
+    //   more, one in it:                256 x 1000 (0.98) 63.5 / 67.3          224 x 1000 (0.86) 61.8 / 66.6
+    //                                   320 x 1000 (0.81) 90.2 / 82.4          256 x 800 (0.78) 51.3 / 48.1
     const int skvp = static_cast<int>(cdiv(a->skv, 32) * 32);
     const bool o_al = aligned(a->o, 8) && ubytes(a->o_stride_nb, es) % 8 == 0 && ubytes(a->o_stride_s, es) % 8 == 0;
     const size_t lds = res_lds_bytes(32, skvp);
     const int64_t blocks = mul_sat({a->nb, a->heads, cdiv(a->sq, 512)});
     const int cus = device_cu_count();
-    if (o_al && cus > 0 && lds <= 150 * 1024 && blocks >= cus && (blocks <= cus || lds <= 80 * 1024))
-      return launch_res(p, skvp, as_stream(stream));
+    if (o_al && cus > 0 && lds <= 150 * 1024) {
+      const double rounds = static_cast<double>(cdiv(blocks, cus));
+      const double filled = static_cast<double>(mul_sat({a->nb, a->heads, a->sq})) / (rounds * cus * 512.0);
+      if (filled >= (blocks <= cus || lds <= 80 * 1024 ? 0.65 : 0.85)) return launch_res(p, skvp, as_stream(stream));
+    }
   }
   if (al) {
     const int32_t rc = a->dtype == WC_F32    ? attn_stream32(p, as_stream(stream))

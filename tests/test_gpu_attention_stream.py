@@ -162,3 +162,22 @@ def test_stream_first_scores_are_minus_infinity(hip, dtype, blocked, causal):
     else:
         ref = (sums[:, -1:] / (s - blocked)).expand(2, s, heads * dh)
     assert _err(got, ref) <= BAR[dtype]
+
+
+@pytest.mark.parametrize("s,heads,fewer", [
+    (1000, 128, 125),             # K and V of one workgroup fill a CU's LDS: a full round, and all but 6 of its places
+    (1000, 256, 230),             # two rounds
+    (512, 256, 200),              # two workgroups share a CU's LDS
+])
+def test_resident_and_streaming_kernels_share_a_range(hip, s, heads, fewer):
+    """bf16, head dim 32: the choice between the resident and the streaming kernel follows how full the chip is, not one
+    number of workgroups: a few heads less take the same kernel (the same bits), and either keeps the bar."""
+    torch.manual_seed(s)
+    q, k, v = (torch.randn(heads, s, 32, device=DEV).to(torch.bfloat16) for _ in range(3))
+    full = _attend(q, k, v, 1, False, False)
+    part = _attend(q[:fewer], k[:fewer], v[:fewer], 1, False, False)
+    few = _attend(q[:20], k[:20], v[:20], 1, False, False)
+    assert torch.equal(part, full[:fewer])
+    ref = _ref(q[:20], k[:20], v[:20], 1, False)
+    for got in (full[:20], few):
+        assert _err(got, ref) <= BAR[torch.bfloat16]
