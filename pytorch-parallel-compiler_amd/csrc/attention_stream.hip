@@ -21,13 +21,14 @@
 //
 // Bound by the VALU: about 51 full-rate instructions and 16 exponentials per 32 x 32 scores
 // against 256 cycles of MFMA at head dim 64; four waves per SIMD (two from head dim 96 on)
-// overlap the two.  Measured (us, heads x tokens x head dim; before: 16x16x32 MFMAs, V transposed
+// overlap the two (causal, 2048 x 64: MFMAs 25 % of the cycles, other VALU instructions 48 %).  Registers: at
+// head dim 64 the full forms spill 4 (eight waves) and 10 (four waves) to stay at four waves per SIMD.  Measured (us, heads x tokens x head dim; before: 16x16x32 MFMAs, V transposed
 // on its way into LDS, a mask and a rescale on every tile):
-//   bf16  64 x 2048 x 64 causal   159  -> 52  (658 TFLOP/s of the lower triangle)
-//   bf16  64 x 2048 x 64          212  -> 92  (749 TFLOP/s)
-//   bf16  32 x 2048 x 128 causal  246  -> 64
-//   bf16  64 x 1024 x 80           94  -> 38.7
-//   fp16  64 x 2048 x 64 causal   159  -> 53.6
+//   bf16  64 x 2048 x 64 causal   159  -> 57.2  (601 TFLOP/s of the lower triangle)
+//   bf16  64 x 2048 x 64          212  -> 100   (687 TFLOP/s)
+//   bf16  32 x 2048 x 128 causal  244  -> 66.8
+//   bf16  64 x 1024 x 80           93  -> 39.4
+//   fp16  64 x 2048 x 64 causal   159  -> 55.0
 #include "wc_attn.h"
 
 #include <type_traits>

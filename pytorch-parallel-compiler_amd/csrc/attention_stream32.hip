@@ -1,7 +1,7 @@
 // Streaming attention in fp32 (softmax(Q K^T * scale) V per (model, batch, head), causal or full),
 // head dims up to 64: the structure of attention_stream.hip on bf16 planes.
 //
-// Q, K, V and P are split into three bf16 planes (v = v0 + v1 + v2, every bit of a normal value) and
+// Q, K, V and P are split into three bf16 planes (v = v0 + v1 + v2, every bit of a value from 2^-110 on) and
 // multiplied as the six plane products of at most second order, the largest in one accumulator and
 // the five small ones in another, so a step of 16 rounds the sum about once.  Six 32x32x16 bf16
 // MFMAs take 3/8 of the fp32 MFMA's time.  K and V tiles of 64 keys are loaded one tile ahead,
@@ -13,14 +13,15 @@
 // 2^-110, computes its queries again on the fp32 MFMA, straight from memory.
 //
 // Bound by the VALU (softmax, splitting P: about 2,000 cycles per wave and tile against 1,536 of
-// MFMAs at head dim 32) and, for short sequences, by the latency of the first loads.  Measured (us,
+// MFMAs at head dim 32; at 128 tokens MFMAs take 25 % of the cycles, other VALU instructions 45 %) and, for
+// short sequences, by the latency of the first loads.  Measured (us,
 // heads x tokens x head dim; before: 16x16x4 fp32 MFMAs, V transposed one value at a time; 2-norm
 // error against fp64 in brackets):
-//   2048 x 128 x 32            57 -> 36    [2.9e-7 -> 1.3e-7]
-//     64 x 2048 x 64          657 -> 374   [8.7e-7 -> 3.5e-7]  (184 TFLOP/s)
-//     64 x 2048 x 64 causal   540 -> 214   [4.0e-7 -> 1.7e-7]
-//    512 x 512 x 32           180 -> 107
-// The fp32 way takes about 5 times as long (64 x 2048 x 64: 372 and then 1,790; the general kernel 657).
+//   2048 x 128 x 32            60 -> 40.5  [2.9e-7 -> 1.3e-7]
+//     64 x 2048 x 64          653 -> 383   [8.7e-7 -> 3.5e-7]  (179 TFLOP/s)
+//     64 x 2048 x 64 causal   538 -> 217   [4.0e-7 -> 1.7e-7]
+//    512 x 512 x 32           179 -> 109
+// With the fp32 pass 64 x 2048 x 64 takes 990 us (small V), 2,150 (infinite keys); the general kernel 653.
 // Registers: no scratch at head dims up to 32, 7 (causal 10) spilled at 64; head dims past 64 (Q and O planes of
 // 128 columns) would spill far more and keep the general kernel.
 #include "wc_attn.h"
@@ -213,8 +214,8 @@ void attn_stream32_kernel(AttnParams p) {
         float pv[8];
 #pragma unroll
         for (int r = 0; r < 8; ++r) {
-          // scaled before the subtraction, as the general kernel rounds it
-          pv[r] = __builtin_amdgcn_exp2f(s[b][8 * j + r] * c - base);
+          // one rounding of the argument (the largest P is 1 to within that of the scaled maximum)
+          pv[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][8 * j + r], c, -base));
           if (r & 1) l1 += pv[r];
           else l0 += pv[r];
         }
@@ -313,7 +314,7 @@ void attn_stream32_kernel(AttnParams p) {
       float l0 = 0.f, l1 = 0.f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float pr = __builtin_amdgcn_exp2f(s[r] * c - base);
+        const float pr = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], c, -base));
         if (r & 1) l1 += pr;
         else l0 += pr;
         const int key = k0 + (r >> 2) * 8 + 4 * eh + (r & 3);

@@ -16,13 +16,14 @@
 // for where they can show: by a result under kPlaneSmall, or an operand of kPlaneBig or more.  (16 models x 8,
 // 64 -> 64, 3x3, 32 x 32: 76 us; a zero filter in every 64: 145 for the look; an infinite or small one: 360.)
 //
-// What bounds it: the MFMAs and, for few taps or channels, staging the input tile (its loads are
-// exposed at every 32-channel chunk but for the other workgroup).  Measured (us; before: the
+// What bounds it, in fp32: the MFMAs (34 % of the cycles at 64 -> 64, 3x3) and the VALU work of splitting (30 %);
+// for few taps or channels, staging the input tile (its loads are exposed at every 32-channel chunk but
+// for the other workgroup).  Measured (us; before: the
 // 16x16x4 fp32 MFMA / 16x16x32 with weight fragments read from L2 by every wave; 2-norm error of
 // fp32 against fp64 in brackets):
-//   fp32  16 models x 8, 64 -> 64, 3x3, 32 x 32    123 -> 68    [4.3e-7 -> 1.3e-7]  (142 TFLOP/s)
-//   fp32   2 x 2, 128 -> 128, 7x7, 40 x 50         322 -> 169   [1.4e-6 -> 4.7e-7]
-//   fp32  32 x 16, 1 -> 16, 3x3, 28 x 28           184 -> 79    [5.7e-8 -> 3.7e-8]
+//   fp32  16 models x 8, 64 -> 64, 3x3, 32 x 32    123 -> 72    [4.3e-7 -> 1.3e-7]  (134 TFLOP/s)
+//   fp32   2 x 2, 128 -> 128, 7x7, 40 x 50         320 -> 170   [1.4e-6 -> 4.7e-7]
+//   fp32  32 x 16, 1 -> 16, 3x3, 28 x 28           182 -> 80    [5.7e-8 -> 3.7e-8]
 //   bf16   8 x 4, 64 -> 128, 3x3 stride 2, 33 x 33  41.6 -> 25.7
 //   bf16  20 x 8, 96 -> 64, 3x3, 56 x 56           131 -> 116   (before: a 256-pixel tile kernel)
 //   fp16  16 x 4, 128 -> 128, 3x3, 32 x 32          83 -> 43

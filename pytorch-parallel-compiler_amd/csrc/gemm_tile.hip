@@ -22,15 +22,16 @@
 // if it finds one recomputes too.  Tracking the largest operand costs 1-2 %; testing each for being
 // small instead cost 2-4, and 4-7 where zeros are common.
 //
-// What bounds it: the MFMAs at the clock that random operands allow (a large bf16 product reaches
-// 1.25 PFLOP/s on this chip, a sixth of which is 208 TFLOP/s in fp32), and for short k the first
-// loads and the epilogue of each tile.  Measured (us, before: the 16x16x4 fp32 MFMA and a 16-bit
+// What bounds it, in fp32: the MFMAs (42 % of the cycles at k = 256) and the VALU work of splitting the
+// operands (about as many), which overlap only between waves; a large bf16 product reaches 1.25 PFLOP/s on
+// this chip at the clock that random operands allow, a sixth of which is 208 TFLOP/s.  In 16 bits, and for
+// short k, the latency of the first loads and the epilogue of each tile (MFMAs 13 % at k = 300).  Measured (us, before: the 16x16x4 fp32 MFMA and a 16-bit
 // kernel with 32-deep K steps whose unaligned rows were loaded one value at a time):
-//   fp32  16 x 2048 x 256 x 1024    204.6 -> 113    (152 TFLOP/s)
-//   fp32   2 x 4096 x 2048 x 2048   633   -> 383    (179 TFLOP/s)
-//   fp32  16 x 2048 x 257 x 1021    276   -> 141
-//   bf16  20 x 800 x 300 x 1000     104   -> 31     (rows of 600 bytes)
-//   bf16   4 x 4096 x 512 x 512      25.7 -> 19.3   (446 TFLOP/s)
+//   fp32  16 x 2048 x 256 x 1024    204   -> 120    (143 TFLOP/s)
+//   fp32   2 x 4096 x 2048 x 2048   633   -> 380    (181 TFLOP/s)
+//   fp32  16 x 2048 x 257 x 1021    276   -> 137
+//   bf16  20 x 800 x 300 x 1000     102   -> 28.5   (rows of 600 bytes)
+//   bf16   4 x 4096 x 512 x 512      25.7 -> 17.5   (490 TFLOP/s)
 // (models x m x k x o).  Error against fp64, 2-norm, fp32: 2.84e-7 -> 2.46e-7 at k = 256,
 // 7.99e-7 -> 6.94e-7 at k = 2048.
 #include "wc_gemm.h"

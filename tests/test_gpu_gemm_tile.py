@@ -79,7 +79,7 @@ def test_tile_gemm_packed_rows(hip):
     _check(y, ref, i)
 
 
-@pytest.mark.parametrize("n,m,o,k", [(130, 128, 128, 64), (200, 64, 64, 40)])
+@pytest.mark.parametrize("n,m,o,k", [(130, 128, 128, 64), (200, 64, 64, 40), (520, 128, 128, 64)])
 def test_tile_gemm_fp32_special_values(hip, n, m, o, k):
     """Infinities, NaN, values above the largest bf16 and overflowing sums give what fp32 arithmetic gives;
     rows without them keep their values to the fp32 bar."""

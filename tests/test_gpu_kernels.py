@@ -576,14 +576,14 @@ class _MLPTap(_MLP):
     (100, 32, 64, 128, 64, True),     # the MLP configuration's shapes
     (7, 37, 32, 64, 16, True),        # rows straddle two 32-row blocks
     (3, 5, 96, 32, 48, False),        # no activation between the layers
-    (4, 9, 20, 40, 12, True),         # sizes the fused kernel does not take: two launches
+    (4, 9, 20, 40, 12, True),         # widths that are no multiple of 16: the any-width kernel
     (5, 100, 64, 96, 128, True),      # fp32: 24-chunk h rows (swizzle over 8), 4 row blocks
-    (3, 40, 128, 192, 128, True),     # bf16: 12 hidden column blocks; fp32 exceeds LDS: two launches
+    (3, 40, 128, 192, 128, True),     # bf16: 12 hidden column blocks; fp32 exceeds that kernel's LDS: any-width
     (8, 1040, 64, 128, 48, True),     # 264 workgroups of 32 rows (the others run 16-row ones);
                                       # 3 output column blocks: one wave's tile is unpaired
 ])
 def test_traced_linear_chain(hip, dtype, n, b, d_in, d_hidden, d_out, relu):
-    """Linear -> [ReLU] -> Linear runs as one wc_mlp2 launch when the sizes allow it."""
+    """Linear -> [ReLU] -> Linear runs as one launch (wc_mlp2 or wc_mlp2_any) when the sizes allow it."""
     import wide_compiler as wc
     models = []
     for i in range(n):
