@@ -298,21 +298,22 @@ void conv_tile_kernel(ConvParams p) {
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int e = 0; e < 16; ++e) bad |= !(__builtin_fabsf(acc[i][e]) <= 3.402823466e38f);
-    bool small = abs_min16(acc[1], abs_min16(acc[0], INFINITY)) < kPlaneSmall;
-    if (__builtin_amdgcn_ballot_w64(small) != 0) {
+    bool small = co0 + cw + l32 < p.co && abs_min16(acc[1], abs_min16(acc[0], INFINITY)) < kPlaneSmall;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(small) != 0, 0)) {
       // of outputs that exist?  The wave's pixels, one a lane; then the lane's own: bit 32 i + 8 q + e
       const int px = px0 + lane, pr = px / p.tc;
       const uint64_t mine = __builtin_amdgcn_ballot_w64(pr < p.tr && ho0 + pr < p.ho && wo0 + px - pr * p.tc < p.wo) >>
                             (4 * hf);
-      small = false;
+      bool real = false;
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int e = 0; e < 16; ++e)
-          small |= __builtin_fabsf(acc[i][e]) < kPlaneSmall && (mine >> (32 * i + 8 * (e >> 2) + (e & 3)) & 1) != 0;
+          real |= __builtin_fabsf(acc[i][e]) < kPlaneSmall && (mine >> (32 * i + 8 * (e >> 2) + (e & 3)) & 1) != 0;
+      small &= real;
     }
     // could an operand under kPlaneMin show?
-    if (top >= kPlaneBig || (small && co0 + cw + l32 < p.co)) flags[0] = 1;
+    if (top >= kPlaneBig || small) flags[0] = 1;
   }
   // ---- bias and folded BN of the lane's channel, into LDS as [channel][pixel] ----
   const int co = co0 + cw + l32;
@@ -330,75 +331,78 @@ void conv_tile_kernel(ConvParams p) {
   }
   __syncthreads();
   if constexpr (PLANES == 3) {
-    // filters: wrow elements per output channel, tap (t, r, s) of channel c at ((t kh + r) kw + s) wts + c wcs
-    const int wrow = RAW ? p.ci * taps : taps_all * p.ci32, wts = RAW ? 1 : p.ci32, wcs = RAW ? taps : 1;
-    const T* const wall = RAW ? wnb : wb + static_cast<int64_t>(co0) * wrow;
-    if (flags[0] != 0) {
-      bool below = false;
-      const int64_t welems = static_cast<int64_t>(p.co - co0 < 64 ? p.co - co0 : 64) * wrow;
-      for (int64_t e = tid * 8; e < welems; e += kConvThreads * 8) {
-        T v[8];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] = e + q < welems ? wall[e + q] : from_f32<T>(0.f);
-        below |= below_planes(v);
-      }
-      for (int t = 0; t < p.kd; ++t) {
-        const int di = od * p.sd - p.pd + t * p.dd;
-        if (di < 0 || di >= p.d) continue;
-        for (int e = tid; e < npix * ((p.ci + 7) / 8); e += kConvThreads) {
-          const int cg = e / npix, rc = e - cg * npix, r = rc / p.ic;
-          const int hi = hi0 + r, wi = wi0 + rc - r * p.ic;
-          const bool in = hi >= 0 && hi < p.h && wi >= 0 && wi < p.w;
-          const T* const xp = xb + static_cast<int64_t>(cg * 8) * p.x_cs + (static_cast<int64_t>(di) * p.h + hi) * p.w + wi;
+    if (__builtin_expect(flags[0] != 0 || __builtin_amdgcn_ballot_w64(bad) != 0, 0)) {
+      // filters: wrow elements per output channel, tap (t, r, s) of channel c at ((t kh + r) kw + s) wts + c wcs
+      const int wrow = RAW ? p.ci * taps : taps_all * p.ci32, wts = RAW ? 1 : p.ci32, wcs = RAW ? taps : 1;
+      const T* const wall = RAW ? wnb : wb + static_cast<int64_t>(co0) * wrow;
+      if (flags[0] != 0) {                             // the same for the whole workgroup
+        bool below = false;
+        const int64_t welems = static_cast<int64_t>(p.co - co0 < 64 ? p.co - co0 : 64) * wrow;
+        for (int64_t e = tid * 8; e < welems; e += kConvThreads * 8) {
           T v[8];
 #pragma unroll
-          for (int q = 0; q < 8; ++q) v[q] = in && cg * 8 + q < p.ci ? xp[q * p.x_cs] : from_f32<T>(0.f);
+          for (int q = 0; q < 8; ++q) v[q] = e + q < welems ? wall[e + q] : from_f32<T>(0.f);
           below |= below_planes(v);
         }
-      }
-      if (below) flags[1] = 1;
-      __syncthreads();
-      bad |= flags[1] != 0;
-    }
-    if (__builtin_amdgcn_ballot_w64(bad) != 0) {
-      // 8 channels of a tap at a time, 4 of each lane half: a step pairs channels c and c + 4.  A padding pixel is
-      // a zero that meets the weight: an infinite weight gives NaN there.
-      const T* const wl = wall + static_cast<int64_t>(co0 + cw + l32 < p.co ? cw + l32 : p.co - 1 - co0) * wrow;
-      int prow[2], pcol[2];
+        for (int t = 0; t < p.kd; ++t) {
+          const int di = od * p.sd - p.pd + t * p.dd;
+          if (di < 0 || di >= p.d) continue;
+          for (int e = tid; e < npix * ((p.ci + 7) / 8); e += kConvThreads) {
+            const int cg = e / npix, rc = e - cg * npix, r = rc / p.ic;
+            const int hi = hi0 + r, wi = wi0 + rc - r * p.ic;
+            const bool in = hi >= 0 && hi < p.h && wi >= 0 && wi < p.w;
+            const T* const xp = xb + static_cast<int64_t>(cg * 8) * p.x_cs +
+                                (static_cast<int64_t>(di) * p.h + hi) * p.w + wi;
+            T v[8];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int px = px0 + i * 32 + l32, pr = px / p.tc;
-        prow[i] = pr < p.tr ? hi0 + pr * p.sh : hi0; // pixels past the tile repeat its first
-        pcol[i] = pr < p.tr ? wi0 + (px - pr * p.tc) * p.sw : wi0;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
-      }
-      for (int t = 0; t < p.kd; ++t) {
-        const int di = od * p.sd - p.pd + t * p.dd;
-        if (di < 0 || di >= p.d) continue;
-        for (int r = 0; r < p.kh; ++r)
-          for (int s = 0; s < p.kw; ++s) {
-            const T* xp[2];
-            bool in[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-              const int hi = prow[i] + r * p.dh, wi = pcol[i] + s * p.dw;
-              in[i] = hi >= 0 && hi < p.h && wi >= 0 && wi < p.w;
-              xp[i] = xb + (static_cast<int64_t>(di) * p.h + hi) * p.w + wi;
-            }
-            const T* const wp = wl + static_cast<int64_t>((t * p.kh + r) * p.kw + s) * wts;
-            for (int c0 = 4 * hf; c0 - 4 * hf < p.ci; c0 += 8)
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                const int c = c0 + e;
-                const float wv = c < p.ci ? to_f32(wp[c * wcs]) : 0.f;
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                  const float xv = c < p.ci && in[i] ? to_f32(xp[i][c * p.x_cs]) : 0.f;
-                  acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(xv, wv, acc[i], 0, 0, 0);
-                }
-              }
+            for (int q = 0; q < 8; ++q) v[q] = in && cg * 8 + q < p.ci ? xp[q * p.x_cs] : from_f32<T>(0.f);
+            below |= below_planes(v);
           }
+        }
+        if (below) flags[1] = 1;
+        __syncthreads();
+        bad |= flags[1] != 0;
+      }
+      if (__builtin_amdgcn_ballot_w64(bad) != 0) {
+        // 8 channels of a tap at a time, 4 of each lane half: a step pairs channels c and c + 4.  A padding pixel is
+        // a zero that meets the weight: an infinite weight gives NaN there.
+        const T* const wl = wall + static_cast<int64_t>(co0 + cw + l32 < p.co ? cw + l32 : p.co - 1 - co0) * wrow;
+        int prow[2], pcol[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int px = px0 + i * 32 + l32, pr = px / p.tc;
+          prow[i] = pr < p.tr ? hi0 + pr * p.sh : hi0; // pixels past the tile repeat its first
+          pcol[i] = pr < p.tr ? wi0 + (px - pr * p.tc) * p.sw : wi0;
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
+        }
+        for (int t = 0; t < p.kd; ++t) {
+          const int di = od * p.sd - p.pd + t * p.dd;
+          if (di < 0 || di >= p.d) continue;
+          for (int r = 0; r < p.kh; ++r)
+            for (int s = 0; s < p.kw; ++s) {
+              const T* xp[2];
+              bool in[2];
+#pragma unroll
+              for (int i = 0; i < 2; ++i) {
+                const int hi = prow[i] + r * p.dh, wi = pcol[i] + s * p.dw;
+                in[i] = hi >= 0 && hi < p.h && wi >= 0 && wi < p.w;
+                xp[i] = xb + (static_cast<int64_t>(di) * p.h + hi) * p.w + wi;
+              }
+              const T* const wp = wl + static_cast<int64_t>((t * p.kh + r) * p.kw + s) * wts;
+              for (int c0 = 4 * hf; c0 - 4 * hf < p.ci; c0 += 8)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                  const int c = c0 + e;
+                  const float wv = c < p.ci ? to_f32(wp[c * wcs]) : 0.f;
+#pragma unroll
+                  for (int i = 0; i < 2; ++i) {
+                    const float xv = c < p.ci && in[i] ? to_f32(xp[i][c * p.x_cs]) : 0.f;
+                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(xv, wv, acc[i], 0, 0, 0);
+                  }
+                }
+            }
+        }
       }
     }
   }
