@@ -28,7 +28,8 @@
 //
 // What the planes do not carry: a workgroup whose W_hh rows, or a step whose h, hold a value of 2^56 or more
 // (kPlaneSafe) or an infinity computes its gates with fp32 multiply-adds from memory instead.  Below it no gate
-// sum overflows, and what the planes lose of a value under 2^-110 stays 2^-60 of a gate's range.
+// sum overflows, and what the planes lose of a value under 2^-110 stays 2^-60 of a gate's range.  (An infinite
+// weight in every model: LSTM 16 x 16 x 64 x 256 whole forward 1,090 us against 222; per-step launches 625.)
 //
 // Bound by the step's serial chain: MFMAs (and the LDS reads that feed them), the store, flag and
 // load latencies of the exchange.  Measured (us; before: one launch per step, streaming W_hh):
@@ -252,15 +253,22 @@ void part32_kernel(P32Params p) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) gh[j][q] = 0.f;
       if (t > 0 || p.h0) {
-        const float* hr = t == 0 ? p.h0 + (mb + (brow ? fr : 0)) * H
-                                 : p.out + ((mb + (brow ? fr : 0)) * p.steps + t - 1) * H;
-        for (int k = 0; k < H; ++k) {
-          const float hk = __hip_atomic_load(hr + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const float* const h0r = t == 0 ? p.h0 + (mb + (brow ? fr : 0)) * H : nullptr;
+        const float* const wr = p.w_hh + (wrow0 + ul) * H;
+        for (int k = 0; k < H; k += 4) {
+          f32x4 hk;
+          if (t == 0) hk = *reinterpret_cast<const f32x4*>(h0r + k);
+          else
+            hk = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ors, ((orow + t - 1) * H + k) * 4, 0,
+                                                                                 kSc1));
 #pragma unroll
           for (int j = 0; j < TPW; ++j)
 #pragma unroll
-            for (int q = 0; q < NG; ++q)
-              gh[j][q] += hk * p.w_hh[(wrow0 + static_cast<int64_t>(q) * H + ul + j) * H + k];
+            for (int q = 0; q < NG; ++q) {
+              const f32x4 w = *reinterpret_cast<const f32x4*>(wr + (static_cast<int64_t>(q) * H + j) * H + k);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) gh[j][q] += hk[e] * w[e];
+            }
         }
       }
     }
